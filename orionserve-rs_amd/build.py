@@ -20,6 +20,7 @@ SOURCES = [
     "attention_prefill.hip",
     "prefill_plan.cpp",
     "gemm.hip",
+    "gemm_rows.hip",
     "elementwise.hip",
     "runtime.cpp",
     "checkpoint.cpp",

@@ -278,7 +278,7 @@ __device__ __forceinline__ void decode_wave_mfma2(
     const uint16_t* __restrict__ kv_layer, uint32_t blk_stride, uint32_t v_off,
     uint32_t slot_stride, uint32_t head_stride, int bs_log2, int num_q_heads, const float* __restrict__ q,
     const uint32_t* __restrict__ tbl, int blk0, int max_splits, float scale,
-    float* __restrict__ out, float* __restrict__ ws_o, float* __restrict__ ws_ml, uint16_t* VL,
+    const AttnOut& out, float* __restrict__ ws_o, float* __restrict__ ws_ml, uint16_t* VL,
     uint16_t* QL, uint16_t* KL, int row, int kvh,
     int start, int end, int split, int nsplit, const int32_t* __restrict__ prow = nullptr) {
   constexpr int QC = G * PR;      // query columns in use
@@ -505,11 +505,14 @@ __device__ __forceinline__ void decode_wave_mfma2(
   const int64_t hidx = (int64_t)orow * num_q_heads + (int64_t)kvh * G + ohead;
   if (nsplit == 1) {
     const float inv = 1.f / lsum;
-    float* op = out + hidx * D + 4 * grp;
 #pragma unroll
-    for (int t = 0; t < DT; ++t)
-      *reinterpret_cast<float4*>(op + 16 * t) =
-          make_float4(o[t][0] * inv, o[t][1] * inv, o[t][2] * inv, o[t][3] * inv);
+    for (int t = 0; t < DT; ++t) {
+      const float4 v = make_float4(o[t][0] * inv, o[t][1] * inv, o[t][2] * inv, o[t][3] * inv);
+      if (out.frag)
+        store_frag4(out.frag, out.mtiles, orow, (kvh * G + ohead) * D + 16 * t + 4 * grp, v);
+      else
+        *reinterpret_cast<float4*>(out.rows + hidx * D + 16 * t + 4 * grp) = v;
+    }
   } else {
     const int64_t slot = hidx * max_splits + split;
     float* op = ws_o + slot * D + 4 * grp;
@@ -537,7 +540,7 @@ __attribute__((amdgpu_waves_per_eu((D == 128 && G * PR > 8) ? 2 : 3)))
                               const int32_t* __restrict__ row_seq,
                               const int64_t* __restrict__ bt_off,
                               const uint32_t* __restrict__ bt_ids, int max_splits,
-                              float scale, float* __restrict__ out, float* __restrict__ ws_o,
+                              float scale, AttnOut out, float* __restrict__ ws_o,
                               float* __restrict__ ws_ml, const int32_t* __restrict__ pack_rows) {
   __shared__ __attribute__((aligned(16))) uint16_t lds_v[4][16 * (D + 8)];
   __shared__ __attribute__((aligned(16))) uint16_t lds_q[4][2 * G * PR * (D + 8)];
@@ -583,7 +586,7 @@ __global__ void __launch_bounds__(256)
                                 const int32_t* __restrict__ row_nsplit,
                                 const int32_t* __restrict__ row_list,
                                 int max_splits, const float* __restrict__ ws_o,
-                                const float* __restrict__ ws_ml, float* __restrict__ out) {
+                                const float* __restrict__ ws_ml, AttnOut out) {
   constexpr int PER = D / 64;
   constexpr int MAXS = 16;
   const int lane = threadIdx.x & 63;
@@ -647,7 +650,14 @@ __global__ void __launch_bounds__(256)
   }
   const float inv = 1.f / lsum;
 #pragma unroll
-  for (int i = 0; i < PER; ++i) out[item * D + lane + 64 * i] = acc[i] * inv;
+  for (int i = 0; i < PER; ++i) {
+    const int d = lane + 64 * i;
+    if (out.frag)
+      store_frag(out.frag, out.mtiles, row, (int)(item - (int64_t)row * num_q_heads) * D + d,
+                 acc[i] * inv);
+    else
+      out.rows[item * D + d] = acc[i] * inv;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -850,7 +860,7 @@ static hipError_t launch_mfma2(int G, dim3 grid, hipStream_t st, const uint16_t*
                                const ArenaStrides& a, int bsl, int hkv, int hq,
                                const DecodeWork* work, int nwork, const float* q,
                                const uint32_t* pos, const int32_t* rs, const int64_t* bo,
-                               const uint32_t* bi, int ms, float scale, float* out,
+                               const uint32_t* bi, int ms, float scale, const AttnOut& out,
                                float* wo, float* wml, const int32_t* pack_rows) {
 #define ORION_MFMA2_CASE(GG)                                                                   \
   case GG:                                                                                     \
@@ -892,7 +902,7 @@ static hipError_t launch_mfma2(int G, dim3 grid, hipStream_t st, const uint16_t*
 // Merges the split-K partials of every row (or of plan.rows) into out.
 static hipError_t launch_combine(hipStream_t st, int64_t D, int64_t rows, int64_t hq,
                                  const DecodePlanDev& plan, int ms, const float* ws_o,
-                                 const float* ws_ml, float* out) {
+                                 const float* ws_ml, const AttnOut& out) {
   const int64_t nr = plan.rows ? plan.num_rows : rows;
   if (nr == 0) return hipSuccess;
   dim3 cgrid((unsigned)((nr * hq + 3) / 4));
@@ -900,7 +910,7 @@ static hipError_t launch_combine(hipStream_t st, int64_t D, int64_t rows, int64_
     if (D > kMaxHeadDim) return hipErrorInvalidValue;
 #define ORION_COMBINE_ANY(NI)                                                                  \
   hipLaunchKernelGGL(paged_decode_combine_any_kernel<NI>, cgrid, dim3(256), 0, st, (int)nr,  \
-                     (int)hq, (int)D, plan.row_nsplit, plan.rows, ms, ws_o, ws_ml, out)
+                     (int)hq, (int)D, plan.row_nsplit, plan.rows, ms, ws_o, ws_ml, out.rows)
     if (D <= 256)
       ORION_COMBINE_ANY(4);
     else if (D <= 512)
@@ -927,14 +937,14 @@ hipError_t launch_split_merge(hipStream_t st, int64_t D, int64_t rows, int64_t h
     return hipErrorInvalidValue;
   const float* ws_o = plan.ws;
   const float* ws_ml = ws_o + rows * hq * ms * D;
-  return launch_combine(st, D, rows, hq, plan, ms, ws_o, ws_ml, out);
+  return launch_combine(st, D, rows, hq, plan, ms, ws_o, ws_ml, AttnOut{out});
 }
 
 hipError_t launch_paged_decode(hipStream_t st, const KvGeom& kv, const void* arena, int64_t layer,
                                const float* q, int64_t rows, int64_t hq,
                                const uint32_t* positions, const int32_t* row_seq,
                                const int64_t* bt_off, const uint32_t* bt_ids,
-                               const DecodePlanDev& plan, float* out, DecodePhase phase) {
+                               const DecodePlanDev& plan, const AttnOut& out, DecodePhase phase) {
   if (rows == 0 || plan.num_work == 0) return hipSuccess;
   const int64_t hkv = kv.num_kv_heads, D = kv.head_dim;
   if (hkv <= 0 || hq % hkv != 0) return hipErrorInvalidValue;
@@ -958,7 +968,8 @@ hipError_t launch_paged_decode(hipStream_t st, const KvGeom& kv, const void* are
   // MFMA B operand's 16 columns) take the MFMA wave; f32 arenas take the VALU
   // wave up to 8; everything else the general wave.
   // packed prefix items exist only for the MFMA wave, pack_r = 16 / G rows
-  const bool mfma = kv.dtype_bf16 && (D == 64 || D == 128) && G <= 16;
+  const bool mfma = decode_mfma(kv, hq);
+  if (out.frag && !mfma) return hipErrorInvalidValue;
   if (plan.num_packed && (!mfma || G > 8 || plan.pack_r != 16 / G || !plan.pack_rows))
     return hipErrorInvalidValue;
   if ((D != 64 && D != 128) || G > (kv.dtype_bf16 ? 16 : 8)) {
@@ -967,7 +978,7 @@ hipError_t launch_paged_decode(hipStream_t st, const KvGeom& kv, const void* are
   hipLaunchKernelGGL((paged_decode_any_kernel<TT, NC>), grid, dim3(256), 0, st,                \
                      static_cast<const TT*>(arena) + layer * a.layer, a.blk, a.v_off, a.slot,  \
                      a.head, bs_log2, (int)hkv, (int)hq, (int)D, plan.work, plan.num_work, q,  \
-                     bt_ids, ms, scale, out, ws_o, ws_ml)
+                     bt_ids, ms, scale, out.rows, ws_o, ws_ml)
 #define ORION_ANY_D(TT)            \
   do {                             \
     if (D <= 256)                  \
@@ -1013,11 +1024,11 @@ hipError_t launch_paged_decode(hipStream_t st, const KvGeom& kv, const void* are
     if (D == 128)
       e = launch_valu<float, 128>(G, grid, st, base, a, bs_log2, (int)hkv, (int)hq, plan.work,
                                   plan.num_work, q, positions, row_seq, bt_off, bt_ids, ms,
-                                  scale, out, ws_o, ws_ml);
+                                  scale, out.rows, ws_o, ws_ml);
     else if (D == 64)
       e = launch_valu<float, 64>(G, grid, st, base, a, bs_log2, (int)hkv, (int)hq, plan.work,
                                  plan.num_work, q, positions, row_seq, bt_off, bt_ids, ms,
-                                 scale, out, ws_o, ws_ml);
+                                 scale, out.rows, ws_o, ws_ml);
     else
       return hipErrorInvalidValue;
   }

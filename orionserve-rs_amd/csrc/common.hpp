@@ -112,6 +112,24 @@ __device__ inline void split1_trunc(float x, uint16_t& hi, uint16_t& lo) {
   lo = (uint16_t)(__float_as_uint(x - __uint_as_float(b & 0xffff0000u)) >> 16);
 }
 
+// The same pair with both terms rounded to nearest even (v_cvt_pk_bf16_f32):
+// two operations more per pair, a quarter of the error (2.5e-6 against 9.8e-6
+// rms, relative) and no bias.  hi is rounded within the finite bf16 range, so
+// no finite x becomes infinite.
+__device__ inline uint32_t pack_bf16_rne(float a, float b) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+__device__ inline void split2_rne(float x0, float x1, uint32_t& hi, uint32_t& lo) {
+#pragma clang fp contract(off)
+  constexpr float kMax = 3.3895313892515355e38f;  // the largest finite bf16
+  hi = pack_bf16_rne(__builtin_amdgcn_fmed3f(x0, -kMax, kMax),
+                     __builtin_amdgcn_fmed3f(x1, -kMax, kMax));
+  lo = pack_bf16_rne(x0 - bf16lo(hi), x1 - bf16hi(hi));
+}
+
 // Split an f32 into hi + lo bf16 terms: hi = rne(x), lo = rne(x - hi).
 // x - hi is exact in f32, so hi + lo carries ~16 significant bits of x.
 __device__ inline void split_bf16(float x, uint16_t& hi, uint16_t& lo) {

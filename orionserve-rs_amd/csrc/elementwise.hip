@@ -10,14 +10,15 @@ namespace orion {
 
 // TransformerModel::embed (transformer.rs:208-223): row gather, bf16 -> f32.
 // Token ids are range-checked on the host before launch.  With `sumsq`, also
-// the row's f64 sums of squares, one slot per 64 consecutive columns (the
-// slots the residual GEMMs leave for the fused RMSNorm of the next GEMM), so
-// layer 0's QKV GEMM applies its norm the same way.  Workgroup (row, y) takes
+// the row's f64 sums of squares, one slot per 64 consecutive columns, for the
+// RMSNorm that layer 0's QKV GEMM applies (the residual GEMMs leave the later
+// layers'), and with `frag` that GEMM's operand.  Workgroup (row, y) takes
 // 64-column chunks 4y .. 4y + 3, one per wave (one load and at most one
 // reduction per wave).
 __global__ void __launch_bounds__(256)
     embed_kernel(const uint32_t* __restrict__ tokens, const uint16_t* __restrict__ table,
-                 int64_t hidden, float* __restrict__ out, double* __restrict__ sumsq) {
+                 int64_t hidden, float* __restrict__ out, double* __restrict__ sumsq,
+                 uint16_t* __restrict__ frag, const float* __restrict__ next_weight) {
   const int64_t row = blockIdx.x;
   const uint16_t* src = table + (int64_t)tokens[row] * hidden;
   float* dst = out + row * hidden;
@@ -27,6 +28,8 @@ __global__ void __launch_bounds__(256)
     const int64_t i = c * 64 + lane;
     const float v = i < hidden ? bf16_to_f32(src[i]) : 0.f;
     if (i < hidden) dst[i] = v;
+    if (frag && i < hidden)
+      store_frag(frag, act_tiles(gridDim.x), (int)row, (int)i, v * next_weight[i]);
     if (sumsq) {
       const double q = wave_sum_f64((double)v * (double)v);
       if (lane == 0) sumsq[row * nslots + c] = q;
@@ -35,12 +38,47 @@ __global__ void __launch_bounds__(256)
 }
 
 hipError_t launch_embed(hipStream_t st, const uint32_t* tokens, int64_t n, const uint16_t* table,
-                        int64_t hidden, float* out, double* sumsq) {
+                        int64_t hidden, float* out, double* sumsq, uint16_t* frag,
+                        const float* next_weight) {
   if (n == 0) return hipSuccess;
   const int64_t nslots = (hidden + 63) >> 6;
   const unsigned gy = (unsigned)std::min<int64_t>((nslots + 3) / 4, 64);
   hipLaunchKernelGGL(embed_kernel, dim3((unsigned)n, gy), dim3(256), 0, st, tokens, table, hidden,
-                     out, sumsq);
+                     out, sumsq, frag, next_weight);
+  return hipGetLastError();
+}
+
+// What launch_gemm_rows needs of an RMSNorm whose rows no residual GEMM left it
+// (the LM head's gathered rows): the f64 sums of squares, one slot per 64
+// columns, and the rows, times the norm weight in fragment order (frag) or
+// gathered as they are (out_rows).  One wave per 64-column chunk, as embed.
+__global__ void __launch_bounds__(256)
+    norm_input_kernel(const float* __restrict__ x, const int32_t* __restrict__ row_index,
+                      const float* __restrict__ weight, int64_t cols, double* __restrict__ sumsq,
+                      uint16_t* __restrict__ frag, float* __restrict__ out_rows) {
+  const int64_t row = blockIdx.x;
+  const float* src = x + (row_index ? row_index[row] : row) * cols;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t nslots = (cols + 63) >> 6;
+  for (int64_t c = (int64_t)blockIdx.y * 4 + wave; c < nslots; c += (int64_t)gridDim.y * 4) {
+    const int64_t i = c * 64 + lane;
+    const float v = i < cols ? src[i] : 0.f;
+    if (i < cols) {
+      if (frag) store_frag(frag, act_tiles(gridDim.x), (int)row, (int)i, v * weight[i]);
+      if (out_rows) out_rows[row * cols + i] = v;
+    }
+    const double q = wave_sum_f64((double)v * (double)v);
+    if (lane == 0) sumsq[row * nslots + c] = q;
+  }
+}
+
+hipError_t launch_norm_input(hipStream_t st, const float* x, const int32_t* row_index,
+                             const float* weight, int64_t rows, int64_t cols, double* sumsq,
+                             uint16_t* frag, float* out_rows) {
+  if (rows == 0) return hipSuccess;
+  const unsigned gy = (unsigned)std::min<int64_t>(((cols + 63) / 64 + 3) / 4, 64);
+  hipLaunchKernelGGL(norm_input_kernel, dim3((unsigned)rows, gy), dim3(256), 0, st, x, row_index,
+                     weight, cols, sumsq, frag, out_rows);
   return hipGetLastError();
 }
 
@@ -168,7 +206,7 @@ __global__ void __launch_bounds__(256)
                       int64_t v_stride, const uint32_t* __restrict__ positions,
                       const int32_t* __restrict__ row_seq, const int64_t* __restrict__ bt_off,
                       const uint32_t* __restrict__ bt_ids, const float* __restrict__ cos_t,
-                      const float* __restrict__ sin_t, GemmPartials qkv) {
+                      const float* __restrict__ sin_t) {
 #pragma clang fp contract(off)
   extern __shared__ float xs[];
   const int64_t row = blockIdx.x;
@@ -181,10 +219,7 @@ __global__ void __launch_bounds__(256)
   const int64_t slot = pos & ((1u << bs_log2) - 1);
   T* kdst = kv_layer + (int64_t)blk * blk_stride + slot * slot_stride + h * head_stride;
 
-  // Inputs come from the q/k/v buffers, or straight from the QKV GEMM's
-  // unreduced partials.
   auto input = [&](int e) {
-    if (qkv.ws) return partial_sum(qkv, row, (int64_t)unit * D + e);
     return is_q ? q_in[row * q_stride + h * D + e]
          : is_k ? k[row * k_stride + h * D + e]
                 : v[row * v_stride + h * D + e];
@@ -209,8 +244,7 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// The same RoPE + KV write for inputs in the q/k/v buffers (the prefill
-// route), vectorised: thread t of a (row, head) takes dims 4t .. 4t+3 and
+// The same RoPE + KV write, vectorised: thread t of a (row, head) takes dims 4t .. 4t+3 and
 // their rotate-half partners 4t + D/2 .. (no LDS, no barrier; the same f32
 // expressions per element as rope_cache_kernel).  One thread per 8 elements,
 // a flat grid over (row, head, t); needs D % 8 == 0 and 16-byte aligned rows.
@@ -286,21 +320,19 @@ hipError_t launch_rope_and_cache(hipStream_t st, const KvGeom& kv, void* arena, 
                                  float* q_out, const float* k, int64_t k_stride, const float* v,
                                  int64_t v_stride, const uint32_t* positions,
                                  const int32_t* row_seq, const int64_t* bt_off,
-                                 const uint32_t* bt_ids, const float* cos_t, const float* sin_t,
-                                 const GemmPartials* qkv_partials) {
+                                 const uint32_t* bt_ids, const float* cos_t, const float* sin_t) {
   if (rows == 0) return hipSuccess;
-  const GemmPartials qp = qkv_partials ? *qkv_partials : GemmPartials{};
   int bs_log2 = 0;
   while ((1 << bs_log2) < kv.block_size) ++bs_log2;
   const ArenaStrides a = arena_strides(kv);
   if (kv.head_dim > kMaxHeadDim || kv.head_dim % 2 || hq + 2 * kv.num_kv_heads > 65535 ||
       rows > INT32_MAX)
     return hipErrorInvalidValue;
-  // Inputs in the q/k/v buffers with 16-byte aligned rows: the vectorised
-  // kernel (one thread per 8 elements instead of one per element).
+  // 16-byte aligned rows: the vectorised kernel (one thread per 8 elements
+  // instead of one per element).
   const int64_t D = kv.head_dim, units = hq + 2 * kv.num_kv_heads;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (!qp.ws && D % 8 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && v_stride % 4 == 0 &&
+  if (D % 8 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && v_stride % 4 == 0 &&
       al16(q_in) && al16(k) && al16(v) && al16(q_out) && al16(cos_t) && al16(sin_t) &&
       al16(arena)) {
     const int64_t threads = rows * units * (D / 8);
@@ -328,13 +360,13 @@ hipError_t launch_rope_and_cache(hipStream_t st, const KvGeom& kv, void* arena, 
     hipLaunchKernelGGL(rope_cache_kernel<uint16_t>, grid, block, lds, st, base,
                        a.blk, a.v_off, a.slot, a.head, bs_log2, (int)hq, (int)kv.num_kv_heads,
                        (int)kv.head_dim, q_in, q_stride, q_out, k, k_stride, v, v_stride,
-                       positions, row_seq, bt_off, bt_ids, cos_t, sin_t, qp);
+                       positions, row_seq, bt_off, bt_ids, cos_t, sin_t);
   } else {
     float* base = static_cast<float*>(arena) + layer * a.layer;
     hipLaunchKernelGGL(rope_cache_kernel<float>, grid, block, lds, st, base,
                        a.blk, a.v_off, a.slot, a.head, bs_log2, (int)hq, (int)kv.num_kv_heads,
                        (int)kv.head_dim, q_in, q_stride, q_out, k, k_stride, v, v_stride,
-                       positions, row_seq, bt_off, bt_ids, cos_t, sin_t, qp);
+                       positions, row_seq, bt_off, bt_ids, cos_t, sin_t);
   }
   return hipGetLastError();
 }

@@ -20,10 +20,7 @@
 #include "kernels.hpp"
 
 #include <algorithm>
-#include <array>
-#include <cstdio>
 #include <cstdlib>
-#include <cstring>
 #include <type_traits>
 #include <utility>
 
@@ -204,13 +201,13 @@ __device__ inline int swz_a(int r) {
 __device__ inline int swz_b(int n) { return (n >> 2) & 3; }
 }  // namespace
 
-// W is either row-major [N, K] (pk.nt == 0) or in the decode GEMM's packed
-// order (launch_gemv_pack with geometry pk): there a 16-column x 32-k MFMA B
-// fragment is one contiguous KiB, lane l's 16 bytes at l * 16, so each of the
-// tile's 8 fragments per k-step is copied to LDS verbatim and read back with
-// one conflict-free ds_read_b128 per lane.
+// W is either row-major [N, K] or in packed order (launch_pack_weights): there
+// a 16-column x 32-k MFMA B fragment is one contiguous KiB, lane l's 16 bytes
+// at l * 16, so each of the tile's fragments per k-step is copied to LDS
+// verbatim and read back with one conflict-free ds_read_b128 per lane.
 struct PackedGeom {
-  int nt = 0, ks = 0, n_tiles = 0;  // columns per decode workgroup / 64, k-steps per slice
+  bool packed = false;
+  int pair_dim = 0, pair_cols = 0;  // packed_column
 };
 
 // HILO: x carried as a truncated hi + lo bf16 pair (two MFMAs, ~16 bits of
@@ -265,25 +262,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
     const int c = (lane & 7) ^ swz_a(r);
     a_src[j] = x + (int64_t)min(m0 + r, M - 1) * K + c * 4;
   }
-  // Packed W: fragment f = wave * 2 + j holds columns n0 + 16 f .. + 16.  Its
-  // chunk (decode workgroup share) within a K slice, and the last fragment
-  // column group the packed copy holds (columns past it are past N anyway).
-  const bool packed = pk.nt > 0;
-  int64_t b_chunk[BJ] = {};
+  // Packed W: fragment f = wave * BJ + j holds columns n0 + 16 f .. + 16
+  // (clamped to the last column tile; columns past it are past N anyway), its
+  // k-steps 512 elements apart.
+  const bool packed = pk.packed;
 #pragma unroll
   for (int j = 0; j < BJ; ++j) {
     if (packed) {
-      const int c16 = min(n0 / 16 + wave * BJ + j, pk.n_tiles * 4 * pk.nt - 1);
-      const int tile = c16 / (4 * pk.nt), rem = c16 - tile * 4 * pk.nt;
-      b_chunk[j] = ((int64_t)tile * 4 + rem / pk.nt) * pk.nt + rem % pk.nt;
-      b_src[j] = w + (int64_t)lane * 8;
+      const int c16 = min(n0 / 16 + wave * BJ + j, (N + 15) / 16 - 1);
+      b_src[j] = w + (int64_t)c16 * (K / kTK) * 512 + lane * 8;
     } else {
       const int r = (wave * BJ + j) * 16 + (lane >> 2);
       const int c = (lane & 3) ^ swz_b(r);
       b_src[j] = w + (int64_t)min(n0 + r, N - 1) * K + c * 8;
     }
   }
-  const int64_t slice_elems = (int64_t)pk.n_tiles * 4 * pk.nt * pk.ks * 512;  // one K slice
+  const int b_step = packed ? 512 : kTK;
   const uint32_t as_base = (uint32_t)(uintptr_t)&As[0][0];
   const uint32_t bs_base = (uint32_t)(uintptr_t)&Bs[0][0];
   auto load_tile = [&](int ks, int buf) {
@@ -291,17 +285,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       lds_load16(a_src[j] + k0, as_base + (uint32_t)(buf * kTM * kTK * 4 + (wave * 4 + j) * 1024));
-    if (packed) {
-      const int slice = ks / pk.ks, step = ks - slice * pk.ks;
 #pragma unroll
-      for (int j = 0; j < BJ; ++j)
-        lds_load16(b_src[j] + slice * slice_elems + (b_chunk[j] * pk.ks + step) * 512,
-                   bs_base + (uint32_t)(buf * TN * kTK * 2 + (wave * BJ + j) * 1024));
-    } else {
-#pragma unroll
-      for (int j = 0; j < BJ; ++j)
-        lds_load16(b_src[j] + k0, bs_base + (uint32_t)(buf * TN * kTK * 2 + (wave * BJ + j) * 1024));
-    }
+    for (int j = 0; j < BJ; ++j)
+      lds_load16(b_src[j] + (int64_t)ks * b_step,
+                 bs_base + (uint32_t)(buf * TN * kTK * 2 + (wave * BJ + j) * 1024));
   };
 
   // ---- fragment read addresses (bytes, buffer 0) ----
@@ -380,16 +367,33 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
   if (partial) {  // one K split: raw sums, reduced by gemm_tiled_reduce_kernel
     float* pz = partial + (int64_t)blockIdx.z * M * N;
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int nt = 0; nt < NTW; ++nt) {
+      const int col = n0 + wn * 16 * NTW + nt * 16 + l16;
+      const int oc = packed_column(col, pk.pair_dim, pk.pair_cols);
 #pragma unroll
-      for (int nt = 0; nt < NTW; ++nt) {
-        const int col = n0 + wn * 16 * NTW + nt * 16 + l16;
+      for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int row = m0 + wm * 64 + mt * 16 + 4 * grp + i;
-          if (row < M && col < N) pz[(int64_t)row * N + col] = acc[mt][nt][i];
+          if (row < M && col < N) pz[(int64_t)row * N + oc] = acc[mt][nt][i];
         }
-      }
+    }
+    return;
+  }
+  if (ep == (int)Epilogue::kStore) {
+#pragma unroll
+    for (int nt = 0; nt < NTW; ++nt) {
+      const int col = n0 + wn * 16 * NTW + nt * 16 + l16;
+      const int oc = packed_column(col, pk.pair_dim, pk.pair_cols);
+      const float b = bias && col < N ? bias[oc] : 0.f;
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int row = m0 + wm * 64 + mt * 16 + 4 * grp + i;
+          if (row < M && col < N) out[(int64_t)row * N + oc] = bias ? acc[mt][nt][i] + b : acc[mt][nt][i];
+        }
+    }
     return;
   }
   if (ep == (int)Epilogue::kAccumulate) {
@@ -433,24 +437,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
       for (int i = 0; i < 4; ++i) {
         const int row = m0 + wm * 64 + mt * 16 + 4 * grp + i;
         const float v = acc[mt][nt][i];
-        if (ep == (int)Epilogue::kSwiGLU) {
-          // Tile columns [0, 8) are gate rows of W, [8, 16) the matching up rows.
-          const float u = __shfl_xor(v, 8);
-          if (l16 < 8 && row < M && col < N) {
-            const float act = v / (1.0f + __expf(-v)) * u;
-            const int c8 = (n0 + wn * 16 * NTW + nt * 16) >> 1;  // a multiple of 8
-            if (out_hilo) {
-              uint16_t h, lo;
-              split1_trunc(act, h, lo);
-              uint16_t* o16 = reinterpret_cast<uint16_t*>(out) + (int64_t)row * N + c8 * 2;
-              o16[l16] = h;
-              o16[8 + l16] = lo;
-            } else {
-              out[(int64_t)row * (N >> 1) + c8 + l16] = act;
-            }
+        // kSwiGLU: tile columns [0, 8) are gate rows of W, [8, 16) the matching
+        // up rows.
+        const float u = __shfl_xor(v, 8);
+        if (l16 < 8 && row < M && col < N) {
+          const float act = v / (1.0f + __expf(-v)) * u;
+          const int c8 = (n0 + wn * 16 * NTW + nt * 16) >> 1;  // a multiple of 8
+          if (out_hilo) {
+            uint16_t h, lo;
+            split1_trunc(act, h, lo);
+            uint16_t* o16 = reinterpret_cast<uint16_t*>(out) + (int64_t)row * N + c8 * 2;
+            o16[l16] = h;
+            o16[8 + l16] = lo;
+          } else {
+            out[(int64_t)row * (N >> 1) + c8 + l16] = act;
           }
-        } else if (row < M && col < N) {
-          out[(int64_t)row * N + col] = bias ? v + bias[col] : v;
         }
       }
     }
@@ -474,8 +475,9 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// Decode-shaped (M <= 64) weight-streaming GEMM, split over K across
-// workgroups.  Workgroup (256 threads) = 4 waves x NT column tiles of 16 =
+// Few rows (M <= 64) of a row-major W, split over K across workgroups: the
+// op-level entry points (a forward's decode GEMMs read packed weights,
+// gemm_rows.hip).  Workgroup (256 threads) = 4 waves x NT column tiles of 16 =
 // 64*NT output columns, over one K slice of KSTEPS k-steps (32 k each).
 //   1. Every wave issues all of its slice's weight loads at once
 //      (KSTEPS x NT 16-byte loads per lane straight into MFMA B fragments),
@@ -491,12 +493,9 @@ template <int MT, int NT, int KSTEPS>
 __global__ void __launch_bounds__(256)
     gemm_gemv_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
                      const float* __restrict__ bias, int M, int N, int K, int ep,
-                     float* __restrict__ out, float* __restrict__ partial,
-                     const double* __restrict__ nsq, int nslots, const float* __restrict__ nw,
-                     float neps, int wpacked) {
+                     float* __restrict__ out, float* __restrict__ partial) {
   constexpr int BN = 64 * NT;
   __shared__ __attribute__((aligned(16))) uint4 xs[2][MT * KSTEPS * 64];  // [hi|lo][frag][lane]
-  __shared__ float nscale[MT * 16];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -507,23 +506,16 @@ __global__ void __launch_bounds__(256)
   const int k0 = blockIdx.y * KSTEPS * 32;
   const int nsteps = min(KSTEPS, (K - k0) >> 5);
 
-  // Load order: the activation slice (and norm inputs) first, the weights
-  // last, so staging the activations and the first MFMAs wait only for the
-  // L2-resident inputs while the weight stream is still arriving (a wave's
-  // loads complete in issue order).
+  // Load order: the activation slice first, the weights last, so staging the
+  // activations waits only for the L2-resident inputs while the weight stream
+  // is still arriving (a wave's loads complete in issue order).
   // 1. activation slice fragments: fragment f = (mt, step), lane l holds row
   //    mt*16 + l%16, k = step*32 + (l/16)*8 .. +8.
   constexpr int FR = MT * KSTEPS * 64 / 256;  // fragments per thread
   static_assert(MT * KSTEPS * 64 % 256 == 0, "fragments must split evenly over the workgroup");
   // Every load below is unconditional (clamped address, value selected
   // afterwards), so the waits can count them in issue order.
-  // Fragment j of a thread is f = wave + 4j, so fragments j and j + KSTEPS/4
-  // cover the same k (next row tile): the norm weight is loaded for the first
-  // KSTEPS/4 only.
-  static_assert(KSTEPS % 4 == 0, "fragments of one k repeat every KSTEPS/4");
-  constexpr int FW = KSTEPS / 4;
-  float4 xa[FR][2], wa[FW][2];
-  const float* nwp = nsq ? nw : x;
+  float4 xa[FR][2];
 #pragma unroll
   for (int j = 0; j < FR; ++j) {
     const int idx = tid + j * 256;
@@ -534,91 +526,25 @@ __global__ void __launch_bounds__(256)
     const float* xp = x + (int64_t)min(row, M - 1) * K + kk;
     xa[j][0] = *reinterpret_cast<const float4*>(xp);
     xa[j][1] = *reinterpret_cast<const float4*>(xp + 4);
-    if (j < FW) {
-      const float* wp = nwp + (nsq ? kk : 0);
-      wa[j][0] = *reinterpret_cast<const float4*>(wp);
-      wa[j][1] = *reinterpret_cast<const float4*>(wp + 4);
-    }
-  }
-  // Fused RMSNorm: the row's f64 sum-of-squares slots, TPR threads per row,
-  // each summing up to kSlotsPerThread consecutive slots (larger rows take
-  // the loop below, after the weights).
-  constexpr int TPR = MT == 1 ? 16 : MT == 2 ? 8 : 4, kSlotsPerThread = 8;
-  const bool early_norm = nsq && nslots <= TPR * kSlotsPerThread;
-  const int spt = (nslots + TPR - 1) / TPR;
-  double sq[kSlotsPerThread];
-  {
-    const int row = tid / TPR, j = tid % TPR;
-    // (x stands in as a readable address when there is nothing to load)
-    const double* sp = early_norm ? nsq + (int64_t)min(row, M - 1) * nslots
-                                  : reinterpret_cast<const double*>(x);
-    const int last = early_norm ? nslots - 1 : 0;
-#pragma unroll
-    for (int i = 0; i < kSlotsPerThread; ++i) {
-      const int slot = j * spt + i;
-      const bool use = early_norm && row < M && i < spt && slot < nslots;
-      const double v = sp[min(slot, last)];
-      sq[i] = use ? v : 0.0;
-    }
   }
 
   // 2. weight loads (clamped column and k-step: unconditional loads)
-  //    in k-step order, so the MFMAs of step s wait only for its loads
-  //    Row-major W: lane (l16, grp) reads W[col][k .. k+8) of its column.
-  //    Packed W (wpacked, launch_gemv_pack): the workgroup's whole share is
-  //    one contiguous chunk, in dispatch order, and a wave load one
-  //    contiguous KiB.
+  //    in k-step order, so the MFMAs of step s wait only for its loads; lane
+  //    (l16, grp) reads W[col][k .. k+8) of its column
   bf16x8 bw[KSTEPS][NT];
   const uint16_t* wrow[NT];
-  int wstep;
-  if (wpacked) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-      wrow[nt] = w + (((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (4 * NT) + wave * NT + nt) *
-                         (KSTEPS * 512) + lane * 8;
-    wstep = 512;
-  } else {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-      wrow[nt] = w + (int64_t)min(n0 + (wave * NT + nt) * 16 + l16, N - 1) * K + k0 + grp * 8;
-    wstep = 32;
-  }
+  for (int nt = 0; nt < NT; ++nt)
+    wrow[nt] = w + (int64_t)min(n0 + (wave * NT + nt) * 16 + l16, N - 1) * K + k0 + grp * 8;
 #pragma unroll
   for (int s2 = 0; s2 < KSTEPS; ++s2)
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
       bw[s2][nt] = __builtin_bit_cast(
-          bf16x8, *reinterpret_cast<const uint4*>(wrow[nt] + min(s2, nsteps - 1) * wstep));
+          bf16x8, *reinterpret_cast<const uint4*>(wrow[nt] + min(s2, nsteps - 1) * 32));
   // nothing that waits for a load may be scheduled above this point
   __builtin_amdgcn_sched_barrier(0);
 
-  // 3. row scales: scale = 1 / sqrt(mean(x^2) + eps), as rmsnorm_kernel
-  //    computes it from the f64 sum; x * scale * weight below keeps rmsnorm's
-  //    order of the two products.
-  {
-    // (computed unconditionally so the slot loads stay ahead of the weights)
-    double t = 0.0;
-#pragma unroll
-    for (int i = 0; i < kSlotsPerThread; ++i) t += sq[i];
-    // TPR consecutive lanes hold one row: fixed-order butterfly
-#pragma unroll
-    for (int o = TPR / 2; o > 0; o >>= 1) t += __shfl_xor(t, o);
-    const int row = tid / TPR;
-    if (early_norm && tid % TPR == 0 && row < MT * 16)
-      nscale[row] = row < M ? (float)(1.0 / sqrt(t / (double)K + (double)neps)) : 0.f;
-  }
-  if (nsq) {
-    if (!early_norm && tid < MT * 16) {
-      float sc = 0.f;
-      if (tid < M) {
-        double t = 0.0;
-        for (int j = 0; j < nslots; ++j) t += nsq[(int64_t)tid * nslots + j];
-        sc = (float)(1.0 / sqrt(t / (double)K + (double)neps));
-      }
-      nscale[tid] = sc;
-    }
-    __syncthreads();
-  }
 #pragma unroll
   for (int j = 0; j < FR; ++j) {
     const int idx = tid + j * 256;
@@ -629,14 +555,6 @@ __global__ void __launch_bounds__(256)
                   xa[j][1].x, xa[j][1].y, xa[j][1].z, xa[j][1].w};
 #pragma unroll
     for (int e = 0; e < 8; ++e) a[e] = live ? a[e] : 0.f;
-    if (nsq) {
-      const float sc = row < M ? nscale[row] : 0.f;
-      const float4* wj = wa[j % FW];
-      const float wv[8] = {wj[0].x, wj[0].y, wj[0].z, wj[0].w,
-                           wj[1].x, wj[1].y, wj[1].z, wj[1].w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) a[e] = a[e] * sc * wv[e];
-    }
     uint4 hv, lv;
     split2_trunc(a[0], a[1], hv.x, lv.x);
     split2_trunc(a[2], a[3], hv.y, lv.y);
@@ -695,8 +613,8 @@ __global__ void __launch_bounds__(256)
     return;
   }
   // Partial tile of this K slice: partial[slice][tile][row][BN], rows < 16*MT.
-  // gemm_gemv_reduce_kernel (or the consumer of deferred partials) sums the
-  // slices in order; the kernel boundary orders the two.
+  // gemm_gemv_reduce_kernel sums the slices in order; the kernel boundary
+  // orders the two.
   const int64_t tile_elems = (int64_t)MT * 16 * BN;
   float* mine = partial + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * tile_elems;
 #pragma unroll
@@ -715,7 +633,7 @@ template <int MT, int NT>
 __global__ void __launch_bounds__(256)
     gemm_gemv_reduce_kernel(const float* __restrict__ partial, int kslices, int n_tiles,
                             const float* __restrict__ bias, int M, int N, int ep,
-                            float* __restrict__ out, double* __restrict__ sumsq) {
+                            float* __restrict__ out) {
   constexpr int BN = 64 * NT;
   const int64_t tile_elems = (int64_t)MT * 16 * BN;
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // over n_tiles * M * BN
@@ -756,22 +674,9 @@ __global__ void __launch_bounds__(256)
     const float u = __shfl_xor(v, 8);
     if ((c & 15) < 8 && col < N)
       out[(int64_t)row * (N >> 1) + ((col & ~15) >> 1) + (c & 7)] = v / (1.0f + __expf(-v)) * u;
-  } else {
-    float nv = 0.f;
-    if (col < N) {
-      if (ep == (int)Epilogue::kAccumulate)
-        nv = pre + v;
-      else
-        nv = bias ? v + pre : v;
-      out[(int64_t)row * N + col] = nv;
-    }
-    // Sum of squares of the updated row, one f64 slot per (row, 64 columns):
-    // a wave covers 64 consecutive columns of one row.
-    if (sumsq) {
-      const double q = wave_sum_f64((double)nv * (double)nv);
-      const int slot = col >> 6, nslots = (N + 63) >> 6;
-      if ((threadIdx.x & 63) == 0 && slot < nslots) sumsq[(int64_t)row * nslots + slot] = q;
-    }
+  } else if (col < N) {
+    out[(int64_t)row * N + col] =
+        ep == (int)Epilogue::kAccumulate ? pre + v : bias ? v + pre : v;
   }
 }
 
@@ -799,20 +704,16 @@ static void launch_skinny(int KW, dim3 grid, hipStream_t st, const float* x, con
 }
 
 namespace {
-// Split-K decode GEMM geometry: NT x 64 columns per workgroup (BN) and KS
-// k-steps of 32 per K slice; the slices are summed by gemm_gemv_reduce_kernel
-// (or by the consumer of deferred partials).  Chosen per shape from M = 32
-// measurements on the config-4 projections:
-//   N <= 4096, K <= 4096 (QKV, O)  NT 1, KS 8 (O: 32 x 8 workgroups)
-//     partials left to the consumer (QKV into RoPE): NT 2, KS 8; narrower
-//     tiles only repeat the norm and activation staging (7.1 -> 9.9 us in the
-//     decode step)
-//   N > 4096 (gate/up, LM head)    NT 2, KS 8
-//   K > 4096 (down)                NT 1, KS 8 (704 workgroups at 3 per CU;
-//     NT 2, KS 16 had 176 at one per CU: decode step 1.690 -> 1.676 ms)
-// Few column tiles want narrow tiles (more workgroups).  ORION_GEMV_NT /
-// ORION_GEMV_KS override every shape (measurement knobs; NT in {1, 2, 4}, KS
-// in {4, 8, 16}).
+// Split-K GEMM geometry for few rows: NT x 64 columns per workgroup (BN) and
+// KS k-steps of 32 per K slice; the slices are summed by
+// gemm_gemv_reduce_kernel.  Few column tiles want narrow tiles (more
+// workgroups).  Chosen per shape from M = 32 measurements:
+//   N <= 4096, K <= 4096  NT 1, KS 8
+//   N > 4096              NT 2, KS 8
+//   K > 4096              NT 1, KS 8 (2048 x 5632: 704 workgroups at 3 per CU;
+//     NT 2, KS 16 had 176 at one per CU, 0.6 us slower)
+// ORION_GEMV_NT / ORION_GEMV_KS override every shape (measurement knobs; NT in
+// {1, 2, 4}, KS in {4, 8, 16}).
 int gemv_knob(const char* name, int a, int b, int c) {
   const char* e = getenv(name);
   const int v = e ? atoi(e) : 0;
@@ -822,44 +723,15 @@ struct GemvShape {
   int mt, nt, ks, n_tiles, kslices;
   size_t ws_bytes;
 };
-GemvShape gemv_shape(int64_t M, int64_t N, int64_t K, bool deferred = false) {
+GemvShape gemv_shape(int64_t M, int64_t N, int64_t K) {
   static const int knob_nt = gemv_knob("ORION_GEMV_NT", 1, 2, 4);
   static const int knob_ks = gemv_knob("ORION_GEMV_KS", 4, 8, 16);
   GemvShape g;
   g.mt = (int)((M + 15) / 16);
-  if (K > 4096) {
-    g.nt = 1, g.ks = 8;
-  } else if (N > 4096) {
-    g.nt = 2, g.ks = 8;
-  } else if (deferred) {
-    g.nt = 2, g.ks = 8;
-  } else {
-    g.nt = 1, g.ks = 8;
-  }
+  g.nt = K <= 4096 && N > 4096 ? 2 : 1;
+  g.ks = 8;
   if (knob_nt) g.nt = knob_nt;
   if (knob_ks) g.ks = knob_ks;
-  // ORION_GEMV_GEOM="defer:NT:KS,longk:NT:KS,wide:NT:KS,other:NT:KS,head:NT:KS"
-  // (any subset): per-group override (measurement knob; NT in {1, 2, 4}, KS
-  // in {4, 8, 16}); "head" (N > 16384, an LM head) refines "wide".
-  static const std::array<std::pair<int, int>, 5> geom = [] {
-    std::array<std::pair<int, int>, 5> r{};
-    const char* e = getenv("ORION_GEMV_GEOM");
-    if (!e) return r;
-    const char* names[5] = {"defer", "longk", "wide", "other", "head"};
-    for (int i = 0; i < 5; ++i) {
-      const char* p = strstr(e, names[i]);
-      int nt = 0, ks = 0;
-      if (p && sscanf(p + strlen(names[i]), ":%d:%d", &nt, &ks) == 2 &&
-          (nt == 1 || nt == 2 || nt == 4) && (ks == 4 || ks == 8 || ks == 16))
-        r[i] = {nt, ks};
-    }
-    return r;
-  }();
-  {
-    int grp = deferred ? 0 : K > 4096 ? 1 : N > 4096 ? 2 : 3;
-    if (grp == 2 && N > 16384 && geom[4].first) grp = 4;
-    if (geom[grp].first) g.nt = geom[grp].first, g.ks = geom[grp].second;
-  }
   g.n_tiles = (int)((N + 64 * g.nt - 1) / (64 * g.nt));
   g.kslices = (int)((K + g.ks * 32 - 1) / (g.ks * 32));
   g.ws_bytes = g.kslices > 1 ? (size_t)g.kslices * g.n_tiles * g.mt * 16 * 64 * g.nt * 4 : 0;
@@ -868,125 +740,40 @@ GemvShape gemv_shape(int64_t M, int64_t N, int64_t K, bool deferred = false) {
 template <int MT, int NT, int KS>
 void launch_gemv_t(const GemvShape& g, hipStream_t st, const float* x, const uint16_t* w,
                    const float* bias, int M, int N, int K, int ep, float* out,
-                   const GemmScratch* sc, const GemmFuse& f, bool reduce) {
+                   const GemmScratch* sc) {
   hipLaunchKernelGGL((gemm_gemv_kernel<MT, NT, KS>),
-                     dim3((unsigned)g.n_tiles, (unsigned)g.kslices), dim3(256), 0, st, x,
-                     f.w_packed ? f.w_packed : w, bias,
-                     M, N, K, ep, out, sc ? sc->ws : nullptr, f.norm_sumsq, f.norm_slots,
-                     f.norm_weight, f.norm_eps, f.w_packed ? 1 : 0);
-  if (g.kslices > 1 && reduce) {
+                     dim3((unsigned)g.n_tiles, (unsigned)g.kslices), dim3(256), 0, st, x, w, bias,
+                     M, N, K, ep, out, sc ? sc->ws : nullptr);
+  if (g.kslices > 1) {
     const int64_t threads = (int64_t)g.n_tiles * M * 64 * NT;
     hipLaunchKernelGGL((gemm_gemv_reduce_kernel<MT, NT>),
                        dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, sc->ws,
-                       g.kslices, g.n_tiles, bias, M, N, ep, out, f.sumsq_out);
+                       g.kslices, g.n_tiles, bias, M, N, ep, out);
   }
 }
 template <int MT, int NT>
 void launch_gemv_nt(const GemvShape& g, hipStream_t st, const float* x, const uint16_t* w,
                     const float* bias, int M, int N, int K, int ep, float* out,
-                    const GemmScratch* sc, const GemmFuse& f, bool reduce) {
+                    const GemmScratch* sc) {
   if (g.ks == 4)
-    launch_gemv_t<MT, NT, 4>(g, st, x, w, bias, M, N, K, ep, out, sc, f, reduce);
+    launch_gemv_t<MT, NT, 4>(g, st, x, w, bias, M, N, K, ep, out, sc);
   else if (g.ks == 16)
-    launch_gemv_t<MT, NT, 16>(g, st, x, w, bias, M, N, K, ep, out, sc, f, reduce);
+    launch_gemv_t<MT, NT, 16>(g, st, x, w, bias, M, N, K, ep, out, sc);
   else
-    launch_gemv_t<MT, NT, 8>(g, st, x, w, bias, M, N, K, ep, out, sc, f, reduce);
+    launch_gemv_t<MT, NT, 8>(g, st, x, w, bias, M, N, K, ep, out, sc);
 }
 template <int MT>
 void launch_gemv(const GemvShape& g, hipStream_t st, const float* x, const uint16_t* w,
                  const float* bias, int M, int N, int K, int ep, float* out,
-                 const GemmScratch* sc, const GemmFuse& f, bool reduce) {
+                 const GemmScratch* sc) {
   if (g.nt == 1)
-    launch_gemv_nt<MT, 1>(g, st, x, w, bias, M, N, K, ep, out, sc, f, reduce);
+    launch_gemv_nt<MT, 1>(g, st, x, w, bias, M, N, K, ep, out, sc);
   else if (g.nt == 4)
-    launch_gemv_nt<MT, 4>(g, st, x, w, bias, M, N, K, ep, out, sc, f, reduce);
+    launch_gemv_nt<MT, 4>(g, st, x, w, bias, M, N, K, ep, out, sc);
   else
-    launch_gemv_nt<MT, 2>(g, st, x, w, bias, M, N, K, ep, out, sc, f, reduce);
+    launch_gemv_nt<MT, 2>(g, st, x, w, bias, M, N, K, ep, out, sc);
 }
 }  // namespace
-
-// One thread per 16-byte unit of the packed layout: unit u = (chunk, step,
-// lane) with chunk = ((slice * n_tiles + tile) * 4 + wave) * NT + nt, i.e.
-// the order in which gemm_gemv_kernel's workgroups (x = column tile, y = K
-// slice), waves, column tiles, k-steps and lanes read it.  Columns past N and
-// k past K are zero.
-__global__ void __launch_bounds__(256)
-    gemv_pack_kernel(const uint16_t* __restrict__ w, int N, int K, int nt, int ks, int n_tiles,
-                     int64_t units, uint4* __restrict__ out) {
-  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (u >= units) return;
-  const int lane = (int)(u & 63);
-  const int64_t q = u >> 6;
-  const int s = (int)(q % ks);
-  const int64_t chunk = q / ks;
-  const int nti = (int)(chunk % nt);
-  const int wave = (int)((chunk / nt) & 3);
-  const int64_t wg = chunk / (4 * nt);
-  const int bx = (int)(wg % n_tiles), by = (int)(wg / n_tiles);
-  const int col = bx * 64 * nt + (wave * nt + nti) * 16 + (lane & 15);
-  const int k = by * ks * 32 + s * 32 + (lane >> 4) * 8;
-  uint4 v = uint4{0u, 0u, 0u, 0u};
-  if (col < N && k < K) v = *reinterpret_cast<const uint4*>(w + (int64_t)col * K + k);
-  out[u] = v;
-}
-
-// The inverse of gemv_pack_kernel: unit u goes back to W[col][k .. k+8).
-__global__ void __launch_bounds__(256)
-    gemv_unpack_kernel(const uint4* __restrict__ in, int N, int K, int nt, int ks, int n_tiles,
-                       int64_t units, uint16_t* __restrict__ w) {
-  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (u >= units) return;
-  const int lane = (int)(u & 63);
-  const int64_t q = u >> 6;
-  const int s = (int)(q % ks);
-  const int64_t chunk = q / ks;
-  const int nti = (int)(chunk % nt);
-  const int wave = (int)((chunk / nt) & 3);
-  const int64_t wg = chunk / (4 * nt);
-  const int bx = (int)(wg % n_tiles), by = (int)(wg / n_tiles);
-  const int col = bx * 64 * nt + (wave * nt + nti) * 16 + (lane & 15);
-  const int k = by * ks * 32 + s * 32 + (lane >> 4) * 8;
-  if (col < N && k < K) *reinterpret_cast<uint4*>(w + (int64_t)col * K + k) = in[u];
-}
-
-size_t gemv_packed_bytes(int64_t N, int64_t K, bool deferred) {
-  if (K % 32 != 0 || K <= 0 || N <= 0) return 0;
-  const GemvShape g = gemv_shape(1, N, K, deferred);
-  return (size_t)g.n_tiles * g.kslices * 4 * g.nt * g.ks * 1024;
-}
-
-hipError_t launch_gemv_pack(hipStream_t st, const uint16_t* w, int64_t N, int64_t K,
-                            bool deferred, uint16_t* out) {
-  if (K % 32 != 0 || K <= 0 || N <= 0 || N > INT32_MAX || K > INT32_MAX)
-    return hipErrorInvalidValue;
-  const GemvShape g = gemv_shape(1, N, K, deferred);
-  const int64_t units = (int64_t)gemv_packed_bytes(N, K, deferred) / 16;
-  hipLaunchKernelGGL(gemv_pack_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st, w,
-                     (int)N, (int)K, g.nt, g.ks, g.n_tiles, units, reinterpret_cast<uint4*>(out));
-  return hipGetLastError();
-}
-
-hipError_t launch_gemv_unpack(hipStream_t st, const uint16_t* packed, int64_t N, int64_t K,
-                              bool deferred, uint16_t* w) {
-  if (K % 32 != 0 || K <= 0 || N <= 0 || N > INT32_MAX || K > INT32_MAX)
-    return hipErrorInvalidValue;
-  const GemvShape g = gemv_shape(1, N, K, deferred);
-  const int64_t units = (int64_t)gemv_packed_bytes(N, K, deferred) / 16;
-  hipLaunchKernelGGL(gemv_unpack_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, st,
-                     reinterpret_cast<const uint4*>(packed), (int)N, (int)K, g.nt, g.ks,
-                     g.n_tiles, units, w);
-  return hipGetLastError();
-}
-
-bool gemm_splitk_fusable(int64_t M, int64_t N, int64_t K) {
-  if (M < 1 || M > 64 || K % 32 != 0 || K > INT32_MAX || N < 1 || N > INT32_MAX) return false;
-  const GemvShape g = gemv_shape(M, N, K);
-  return g.kslices > 1 && g.kslices <= 65535;
-}
-
-int gemm_sumsq_slots(int64_t N) {
-  return (int)((N + 63) / 64);
-}
 
 // K splits of the LDS-tiled GEMM.  A call with fewer output tiles than CUs
 // leaves CUs idle, so its K is split until the tiles x splits reach
@@ -1033,19 +820,13 @@ void gemm_scratch_need(int64_t M, int64_t N, int64_t K, size_t* ws_bytes, bool p
     if (s > 1) *ws_bytes = (size_t)s * (size_t)M * (size_t)N * sizeof(float);
     return;
   }
-  const GemvShape g = gemv_shape(M, N, K), gd = gemv_shape(M, N, K, true);
-  *ws_bytes = std::max(g.ws_bytes, gd.ws_bytes);
+  *ws_bytes = gemv_shape(M, N, K).ws_bytes;
 }
 
 hipError_t launch_gemm(hipStream_t st, const float* x, const uint16_t* w, const float* bias,
                        int64_t M, int64_t N, int64_t K, Epilogue ep, float* out,
                        const GemmScratch* scratch, const GemmFuse* fuse) {
   const GemmFuse f = fuse ? *fuse : GemmFuse{};
-  if (f.defer) *f.defer = GemmPartials{};
-  const bool needs_splitk = f.norm_sumsq || f.sumsq_out;
-  if (needs_splitk && (!gemm_splitk_fusable(M, N, K) || (f.sumsq_out && ep != Epilogue::kAccumulate) ||
-                       (f.norm_sumsq && (!f.norm_weight || f.norm_slots < 1))))
-    return hipErrorInvalidValue;
   if (M == 0 || N == 0) return hipSuccess;
   if (K % 32 != 0 || K == 0) return hipErrorInvalidValue;
   if (ep == Epilogue::kSwiGLU && N % 16 != 0) return hipErrorInvalidValue;
@@ -1057,31 +838,18 @@ hipError_t launch_gemm(hipStream_t st, const float* x, const uint16_t* w, const 
   // split-layout activations exist only for the LDS-tiled kernel
   if ((f.x_hilo || f.out_hilo) && (M <= 64 || (M < tiled_min_m && !f.w_packed)))
     return hipErrorInvalidValue;
-  // Decode-shaped M: split-K weight streaming (needs the scratch when K spans
+  // Few rows: split-K weight streaming (needs the scratch when K spans
   // several slices).
-  if (M <= 64 && N <= INT32_MAX && K <= INT32_MAX) {
-    // A consumer that takes the unreduced partials gets them (no reduce
-    // launch); only for the store epilogue.
-    const bool wants_defer = f.defer && ep == Epilogue::kStore && !f.sumsq_out;
-    const GemvShape g = gemv_shape(M, N, K, wants_defer);
+  if (M <= 64 && !f.w_packed && N <= INT32_MAX && K <= INT32_MAX) {
+    const GemvShape g = gemv_shape(M, N, K);
     const bool fits = g.kslices == 1 || (scratch && scratch->ws_bytes >= g.ws_bytes);
-    if (needs_splitk && !fits) return hipErrorInvalidValue;
     if (fits && g.kslices <= 65535) {
       const int m = (int)M, n = (int)N, k = (int)K, e = (int)ep;
-      const bool deferred = wants_defer && g.kslices > 1;
-      if (deferred) {
-        f.defer->ws = scratch->ws;
-        f.defer->kslices = g.kslices;
-        f.defer->n_tiles = g.n_tiles;
-        f.defer->bn = 64 * g.nt;
-        f.defer->tile_rows = g.mt * 16;
-        f.defer->bias = bias;
-      }
       switch (g.mt) {
-        case 1: launch_gemv<1>(g, st, x, w, bias, m, n, k, e, out, scratch, f, !deferred); break;
-        case 2: launch_gemv<2>(g, st, x, w, bias, m, n, k, e, out, scratch, f, !deferred); break;
-        case 3: launch_gemv<3>(g, st, x, w, bias, m, n, k, e, out, scratch, f, !deferred); break;
-        default: launch_gemv<4>(g, st, x, w, bias, m, n, k, e, out, scratch, f, !deferred); break;
+        case 1: launch_gemv<1>(g, st, x, w, bias, m, n, k, e, out, scratch); break;
+        case 2: launch_gemv<2>(g, st, x, w, bias, m, n, k, e, out, scratch); break;
+        case 3: launch_gemv<3>(g, st, x, w, bias, m, n, k, e, out, scratch); break;
+        default: launch_gemv<4>(g, st, x, w, bias, m, n, k, e, out, scratch); break;
       }
       return hipGetLastError();
     }
@@ -1091,11 +859,11 @@ hipError_t launch_gemm(hipStream_t st, const float* x, const uint16_t* w, const 
   if (M >= tiled_min_m || f.w_packed) {
     if (M > (int64_t)65535 * kTM || N > INT32_MAX || K > INT32_MAX) return hipErrorInvalidValue;
     PackedGeom pk;
-    if (f.w_packed) {
-      const GemvShape gp = gemv_shape(1, N, K, f.w_packed_deferred);
-      pk.nt = gp.nt;
-      pk.ks = gp.ks;
-      pk.n_tiles = gp.n_tiles;
+    pk.packed = f.w_packed != nullptr;
+    if (pk.packed) {
+      if (f.pair_dim && ep != Epilogue::kStore) return hipErrorInvalidValue;
+      pk.pair_dim = (int)f.pair_dim;
+      pk.pair_cols = (int)f.pair_cols;
     }
     // 128 x 256 workgroup tiles (64 x 128 per wave, 2 workgroups per CU) for
     // wide outputs: per MFMA a third less LDS traffic (copies + fragment

@@ -3,6 +3,9 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#ifdef __HIPCC__
+#include "common.hpp"
+#endif
 #include <cstddef>
 #include <cstdint>
 #include <vector>
@@ -107,6 +110,14 @@ void build_decode_plan(const uint32_t* positions, const int32_t* row_seq,
 size_t decode_workspace_bytes(int64_t rows, int64_t hq, int64_t D, int64_t max_splits);
 // Rows per packed prefix item for this arena and grouping (0: no packing).
 int decode_pack_rows(const KvGeom& kv, int64_t hq);
+// Where a decode pass writes its rows: f32 rows [row][hq * d], or fragment
+// order over mtiles row tiles (frag set; the MFMA wave's shapes only,
+// decode_mfma).
+struct AttnOut {
+  float* rows = nullptr;
+  uint16_t* frag = nullptr;
+  int mtiles = 0;
+};
 // Which launches of a decode pass to issue (the merge only runs when the
 // plan splits some row).
 enum class DecodePhase { kBoth, kSplit, kMerge };
@@ -116,11 +127,17 @@ enum class DecodePhase { kBoth, kSplit, kMerge };
 // parts use it too).
 hipError_t launch_split_merge(hipStream_t st, int64_t D, int64_t rows, int64_t hq,
                               const DecodePlanDev& plan, float* out);
+// Whether launch_paged_decode runs this shape on the MFMA wave (bf16 arenas at
+// head_dim 64/128, up to 16 query heads per KV head).
+inline bool decode_mfma(const KvGeom& kv, int64_t hq) {
+  return kv.dtype_bf16 && (kv.head_dim == 64 || kv.head_dim == 128) &&
+         hq / kv.num_kv_heads <= 16;
+}
 hipError_t launch_paged_decode(hipStream_t st, const KvGeom& kv, const void* arena, int64_t layer,
                                const float* q, int64_t rows, int64_t hq,
                                const uint32_t* positions, const int32_t* row_seq,
                                const int64_t* bt_off, const uint32_t* bt_ids,
-                               const DecodePlanDev& plan, float* out,
+                               const DecodePlanDev& plan, const AttnOut& out,
                                DecodePhase phase = DecodePhase::kBoth);
 
 // Prefill work list: one entry per (sequence, tile of packed rows, part of
@@ -185,87 +202,128 @@ enum class Epilogue : int {
   kSwiGLU = 2,      // W rows interleaved in groups of 8 gate / 8 up rows;
                     // out[:, N/2] = silu(gate) * up
 };
-// K-slice partial tiles a split-K decode GEMM left unreduced for its consumer
-// to sum (ws == nullptr: the GEMM wrote its output).  Element (row, col) =
-// bias[col] (if any) + sum over slices ks, in slice order, of
-// ws[((ks * n_tiles + col / bn) * tile_rows + row) * bn + col % bn].
-struct GemmPartials {
-  const float* ws = nullptr;
-  int kslices = 0, n_tiles = 0, bn = 0, tile_rows = 0;
-  const float* bias = nullptr;
-};
+// Activations of a decode-shaped forward in fragment order: the layout in
+// which gemm_rows_kernel's lanes read them.  For 16-row tile mt of mtiles,
+// k-step s of 32 and half h (0: the value rounded to bf16, 1: the remainder
+// rounded to bf16; split2_rne) one KiB, lane l's 16 bytes (row 16 mt + l % 16, k
+// 32 s + 8 (l / 16) .. + 8) at 16 l.  Rows are padded to 16; the bytes are
+// those of f32.  Used past kFragMinRows rows (below, f32 rows are fewer bytes
+// than a padded tile).
+constexpr int64_t kFragMinRows = 9;
+__host__ __device__ constexpr int act_tiles(int64_t rows) { return (int)((rows + 15) / 16); }
+inline size_t act_frag_bytes(int64_t rows, int64_t cols) {
+  return (size_t)act_tiles(rows) * 16 * (size_t)((cols + 31) / 32 * 32) * 4;
+}
 #ifdef __HIPCC__
-__device__ inline float partial_sum(const GemmPartials& p, int64_t row, int64_t col) {
-  const int64_t tile = col / p.bn, c = col - tile * p.bn;
-  const float* e = p.ws + (tile * p.tile_rows + row) * p.bn + c;
-  const int64_t stride = (int64_t)p.n_tiles * p.tile_rows * p.bn;
-  // Slices are loaded 8 at a time with every load of a group in flight, then
-  // added in slice order (a slice past the end adds +0, which leaves the sum
-  // unchanged).
-  const float bias = p.bias ? p.bias[col] : 0.f;
-  float v = 0.f;
-  for (int ks0 = 0; ks0 < p.kslices; ks0 += 8) {
-    float t[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) t[j] = ks0 + j < p.kslices ? e[(ks0 + j) * stride] : 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v += t[j];
-  }
-  return p.bias ? v + bias : v;
+// Element (row, col) of half 0, in 2-byte units; half 1 is 512 further on.
+__device__ inline int64_t frag_at(int mtiles, int row, int col) {
+  return ((int64_t)(col >> 5) * mtiles + (row >> 4)) * 1024 +
+         (((col >> 3) & 3) * 16 + (row & 15)) * 8 + (col & 7);
+}
+__device__ inline void store_frag(uint16_t* frag, int mtiles, int row, int col, float v) {
+  uint32_t h, l;
+  split2_rne(v, 0.f, h, l);
+  const int64_t at = frag_at(mtiles, row, col);
+  frag[at] = (uint16_t)h;
+  frag[at + 512] = (uint16_t)l;
+}
+// Four consecutive columns, col a multiple of 4.
+__device__ inline void store_frag4(uint16_t* frag, int mtiles, int row, int col, float4 v) {
+  uint2 h, l;
+  split2_rne(v.x, v.y, h.x, l.x);
+  split2_rne(v.z, v.w, h.y, l.y);
+  const int64_t at = frag_at(mtiles, row, col);
+  *reinterpret_cast<uint2*>(frag + at) = h;
+  *reinterpret_cast<uint2*>(frag + at + 512) = l;
 }
 #endif
+// Column `col` of a packed QKV matrix in W's own order: within the Q and K
+// heads (columns below pair_cols, pair_dim each) a 16-column tile holds 8
+// columns of the head's first half and the 8 of its second half that RoPE
+// rotates them with.  pair_dim 0: W's order.
+__host__ __device__ inline int packed_column(int col, int64_t pair_dim, int64_t pair_cols) {
+  if (!pair_dim || col >= pair_cols) return col;
+  const int D = (int)pair_dim, head = col / D, q = col - head * D;
+  const int e = q & 15, j = (q >> 4) * 8 + (e & 7);
+  return head * D + (e < 8 ? j : (D >> 1) + j);
+}
+// Weights [N, K] in packed order, the layout every GEMM of a forward reads:
+// per 16 columns and 32 k one KiB (an MFMA B fragment, lane l's 16 bytes at
+// 16 l), the k-steps of a column tile consecutive.  0 bytes: K not a multiple
+// of 32.
+size_t packed_weight_bytes(int64_t N, int64_t K);
+hipError_t launch_pack_weights(hipStream_t st, const uint16_t* w, int64_t N, int64_t K,
+                               int64_t pair_dim, int64_t pair_cols, uint16_t* out);
+hipError_t launch_unpack_weights(hipStream_t st, const uint16_t* packed, int64_t N, int64_t K,
+                                 int64_t pair_dim, int64_t pair_cols, uint16_t* w);
 
-// Scratch for split-K decode GEMMs: the K-slice partial tiles.
-struct GemmScratch {
-  float* ws = nullptr;
-  size_t ws_bytes = 0;
+// RoPE and the KV write of a QKV GEMM's rows (launch_rope_and_cache's work):
+// q_out null when the GEMM stores its output instead.  kv is the layer's
+// arena, strides in elements.
+struct RopeOut {
+  float* q_out = nullptr;  // [rows, hq * d]
+  void* kv = nullptr;
+  bool kv_bf16 = false;
+  int hq = 0, hkv = 0, bs_log2 = 0;
+  int64_t blk = 0, v_off = 0, slot = 0, head = 0;
+  const uint32_t* positions = nullptr;
+  const int32_t* row_seq = nullptr;
+  const int64_t* bt_off = nullptr;
+  const uint32_t* bt_ids = nullptr;
+  const float* cos = nullptr;
+  const float* sin = nullptr;
 };
-// Fusions a decode-shaped split-K GEMM (gemm_splitk_fusable) performs with
-// its neighbours, so the RMSNorm and residual-add launches between the layer's
-// GEMMs disappear:
-//  - norm_*: x is the residual stream, and the GEMM multiplies
-//    rms_norm(x[row]) * norm_weight, with the row's scale taken from the
-//    per-row f64 sum-of-squares slots [row][norm_slots] a previous GEMM wrote
-//    (summed in slot order) -- the same per-element roundings as rmsnorm;
-//  - sumsq_out (kAccumulate): after out += x W^T, the GEMM writes the f64 sum
-//    of squares of each updated row in gemm_sumsq_slots(N) slots per row
-//    (slot j covers columns 64j .. 64j+63);
-//  - defer (kStore): the K-slice partials are left unreduced for the consumer
-//    (launch_rope_and_cache) instead of a reduce launch.
-struct GemmFuse {
+// A projection of a decode-shaped forward (gemm_rows.hip) on packed weights.
+struct RowsGemm {
+  const float* x = nullptr;  // f32 rows, or fragment order (x_frag)
+  bool x_frag = false;
+  const uint16_t* w = nullptr;
+  const float* bias = nullptr;  // kStore
+  int64_t M = 0, N = 0, K = 0;
+  Epilogue ep = Epilogue::kStore;
+  float* out = nullptr;
+  // RMSNorm of x: the row sums of squares a previous kernel left
+  // ([row][norm_slots] f64), and for f32 rows the norm weight (fragments
+  // carry it multiplied in)
   const double* norm_sumsq = nullptr;
   int norm_slots = 0;
   const float* norm_weight = nullptr;
   float norm_eps = 0.f;
-  double* sumsq_out = nullptr;
-  GemmPartials* defer = nullptr;
-  // The same weights in the decode kernel's packed order (launch_gemv_pack with
-  // this shape and w_packed_deferred); read instead of w by the decode-shaped
-  // split-K kernel and the LDS-tiled kernel (which then also takes M in
-  // (64, 256)).  w may be null when w_packed is given.
+  // kSwiGLU: the output in fragment order instead of `out`.  kAccumulate: the
+  // updated row times next_weight in fragment order, beside `out`.
+  uint16_t* out_frag = nullptr;
+  const float* next_weight = nullptr;
+  double* sumsq_out = nullptr;  // kAccumulate: rows_sumsq_slots(N) f64 per row
+  // QKV: the packed order of its columns, and the fused RoPE + KV write
+  int64_t pair_dim = 0, pair_cols = 0;
+  RopeOut rope;
+  float* partial = nullptr;  // set by launch_gemm_rows
+};
+constexpr int64_t kRowsMax = 64;  // most rows of a launch_gemm_rows call
+inline int rows_sumsq_slots(int64_t N) { return (int)((N + 15) / 16); }
+size_t rows_scratch_bytes(const RowsGemm& g);
+hipError_t launch_gemm_rows(hipStream_t st, const RowsGemm& g, float* scratch,
+                            size_t scratch_bytes);
+
+// Scratch for split-K GEMMs: the K-slice partial tiles.
+struct GemmScratch {
+  float* ws = nullptr;
+  size_t ws_bytes = 0;
+};
+// What a forward's prefill-shaped GEMMs add to a launch_gemm call (M > 64).
+struct GemmFuse {
+  // the weights in packed order (launch_pack_weights), read instead of w; for
+  // QKV also the order of its columns
   const uint16_t* w_packed = nullptr;
-  bool w_packed_deferred = false;
-  // The LDS-tiled kernel only (M > 64): x arrives already split into its
-  // bf16 hi/lo pair (the layout launch_rmsnorm and the SwiGLU epilogue write
-  // with `hilo`: per row, K/8 groups of [8 hi bf16 | 8 lo bf16], the same
-  // bytes as f32), and a SwiGLU output is written that way.
+  int64_t pair_dim = 0, pair_cols = 0;
+  // x arrives already split into its bf16 hi/lo pair (the layout
+  // launch_rmsnorm and the SwiGLU epilogue write with `hilo`: per row, K/8
+  // groups of [8 hi bf16 | 8 lo bf16], the same bytes as f32), and a SwiGLU
+  // output is written that way.
   bool x_hilo = false;
   bool out_hilo = false;
 };
-// Bytes of W [N, K] in the decode kernel's packed order (0: K not a multiple
-// of 32), and the kernel that writes it from row-major W.  `deferred` must be
-// what the consuming launch_gemm calls will have (GemmFuse::defer set, store
-// epilogue, no sums of squares).
-size_t gemv_packed_bytes(int64_t N, int64_t K, bool deferred);
-hipError_t launch_gemv_pack(hipStream_t st, const uint16_t* w, int64_t N, int64_t K,
-                            bool deferred, uint16_t* out);
-// The inverse: row-major W [N, K] from its packed copy.
-hipError_t launch_gemv_unpack(hipStream_t st, const uint16_t* packed, int64_t N, int64_t K,
-                              bool deferred, uint16_t* w);
-bool gemm_splitk_fusable(int64_t M, int64_t N, int64_t K);
-int gemm_sumsq_slots(int64_t N);
 
-// Scratch a launch_gemm of this shape needs (0 / 0: none).
 // Scratch a launch_gemm call of this shape uses: the decode GEMMs' K-slice
 // partials, or the LDS-tiled GEMM's K-split sums (launch_gemm leaves a tiled
 // GEMM unsplit when the scratch it is given is smaller).
@@ -293,10 +351,20 @@ hipError_t launch_sample(hipStream_t st, float* logits, int64_t rows, int64_t vo
                          int32_t* out);
 
 // ---- elementwise / normalisation -------------------------------------------
-// sumsq: when set, also the row sums of squares in the residual GEMMs' slot
-// layout (gemm_sumsq_slots(hidden) f64 per row).
+// sumsq: when set, also the row sums of squares, one f64 per 64 columns
+// (embed_sumsq_slots(hidden) per row); frag: when set, also the rows times
+// next_weight in fragment order.
+inline int embed_sumsq_slots(int64_t hidden) { return (int)((hidden + 63) / 64); }
 hipError_t launch_embed(hipStream_t st, const uint32_t* tokens, int64_t n, const uint16_t* table,
-                        int64_t hidden, float* out, double* sumsq = nullptr);
+                        int64_t hidden, float* out, double* sumsq = nullptr,
+                        uint16_t* frag = nullptr, const float* next_weight = nullptr);
+// The input of a launch_gemm_rows call that applies an RMSNorm, from f32 rows
+// (gathered by row_index when given): embed_sumsq_slots(cols) sums of squares
+// per row and, when set, the rows times weight in fragment order or a copy of
+// the rows.
+hipError_t launch_norm_input(hipStream_t st, const float* x, const int32_t* row_index,
+                             const float* weight, int64_t rows, int64_t cols, double* sumsq,
+                             uint16_t* frag, float* out_rows);
 // rows selected by `row_index` (nullptr = identity)
 // hilo: out holds each row as cols/8 groups of [8 hi bf16 | 8 lo bf16] (hi =
 // the f32 value truncated to bf16, lo = the remainder truncated), the input
@@ -304,16 +372,12 @@ hipError_t launch_embed(hipStream_t st, const uint32_t* tokens, int64_t n, const
 hipError_t launch_rmsnorm(hipStream_t st, const float* x, const int32_t* row_index,
                           const float* weight, int64_t rows, int64_t cols, float eps, float* out,
                           bool hilo = false);
-// hidden[r] += (deferred GEMM output)[r], then out = rms_norm(hidden[r]) (the
-// residual add of transformer.rs:328-345 fused with the next norm).  With
-// row_index, only the gathered rows are computed and hidden is not written.
 hipError_t launch_rope_and_cache(hipStream_t st, const KvGeom& kv, void* arena, int64_t layer,
                                  int64_t rows, int64_t hq, const float* q_in, int64_t q_stride,
                                  float* q_out, const float* k, int64_t k_stride, const float* v,
                                  int64_t v_stride, const uint32_t* positions,
                                  const int32_t* row_seq, const int64_t* bt_off,
-                                 const uint32_t* bt_ids, const float* cos_t, const float* sin_t,
-                                 const GemmPartials* qkv_partials = nullptr);
+                                 const uint32_t* bt_ids, const float* cos_t, const float* sin_t);
 hipError_t launch_silu_mul(hipStream_t st, float* gate, const float* up, int64_t count);
 hipError_t launch_argmax(hipStream_t st, const float* logits, int64_t rows, int64_t cols,
                          int64_t* out);

@@ -224,8 +224,8 @@ struct LayerDev {
   uint16_t* w_o = nullptr;    // [hidden, Hq*d]
   uint16_t* w_gu = nullptr;   // [2*ffn, hidden], gate/up rows interleaved by 8
   uint16_t* w_down = nullptr; // [hidden, ffn]
-  // The same four matrices in the decode GEMM's packed order (launch_gemv_pack),
-  // which every GEMM of a forward reads.  The row-major ones above exist only
+  // The same four matrices in packed order (launch_pack_weights), which every
+  // GEMM of a forward reads.  The row-major ones above exist only
   // while weights are written or read back (ensure_rowmajor / release_rowmajor).
   uint16_t* p_qkv = nullptr;
   uint16_t* p_o = nullptr;
@@ -237,6 +237,7 @@ struct orion_hip_model {
   orion_hip_device* dev = nullptr;
   orion_hip_model_desc desc{};
   int64_t qd = 0, kvd = 0, qkvd = 0;
+  int64_t pair_dim = 0;  // packed_column of the QKV matrices (0: W's order)
   KvGeom kv{};
   std::vector<void*> allocations;
   std::vector<size_t> alloc_bytes;
@@ -545,6 +546,15 @@ static hipError_t gemm_scratch(orion_hip_device* dev, int64_t M, int64_t N, int6
   return hipSuccess;
 }
 
+static hipError_t gemm_rows_on(orion_hip_device* dev, const RowsGemm& g) {
+  const size_t need = rows_scratch_bytes(g);
+  if (need > dev->gemm_ws.bytes) {
+    hipError_t e = dev->gemm_ws.reserve(need);
+    if (e != hipSuccess) return e;
+  }
+  return launch_gemm_rows(dev->stream, g, dev->gemm_ws.as<float>(), dev->gemm_ws.bytes);
+}
+
 static hipError_t gemm_on(orion_hip_device* dev, const float* x, const uint16_t* w,
                           const float* bias, int64_t M, int64_t N, int64_t K, Epilogue ep,
                           float* out, const GemmFuse* fuse = nullptr) {
@@ -597,6 +607,8 @@ ORION_EXPORT int orion_hip_model_create(orion_hip_device* dev, const orion_hip_m
   m->qd = (int64_t)d.num_attention_heads * d.head_dim;
   m->kvd = (int64_t)d.num_kv_heads * d.head_dim;
   m->qkvd = m->qd + 2 * m->kvd;
+  // (a 16-column tile holds 8 + 8 rotating columns when heads are whole tiles)
+  m->pair_dim = d.head_dim % 16 == 0 ? d.head_dim : 0;
   // Block-internal KV layout of the arena: the reference order unless
   // ORION_KV_LAYOUT=head-major (read at model creation; both measure the same
   // on the decode and prefill kernels).
@@ -1310,45 +1322,43 @@ struct MatrixRef {
   uint16_t** rowmajor;
   uint16_t** packed;
   int64_t N, K;
-  bool deferred;  // QKV: its partials go to RoPE unreduced
+  int64_t pair_dim, pair_cols;  // packed_column (QKV)
 };
 static std::vector<MatrixRef> matrices(orion_hip_model* m) {
   const auto& d = m->desc;
   const int64_t H = d.hidden_size, F = d.intermediate_size, V = d.vocab_size;
   std::vector<MatrixRef> v;
   for (LayerDev& L : m->layers) {
-    v.push_back({&L.w_qkv, &L.p_qkv, m->qkvd, H, true});
-    v.push_back({&L.w_o, &L.p_o, H, m->qd, false});
-    v.push_back({&L.w_gu, &L.p_gu, 2 * F, H, false});
-    v.push_back({&L.w_down, &L.p_down, H, F, false});
+    v.push_back({&L.w_qkv, &L.p_qkv, m->qkvd, H, m->pair_dim, m->qd + m->kvd});
+    v.push_back({&L.w_o, &L.p_o, H, m->qd, 0, 0});
+    v.push_back({&L.w_gu, &L.p_gu, 2 * F, H, 0, 0});
+    v.push_back({&L.w_down, &L.p_down, H, F, 0, 0});
   }
-  if (!d.tied_lm_head) v.push_back({&m->w_lm, &m->p_head, V, H, false});
+  if (!d.tied_lm_head) v.push_back({&m->w_lm, &m->p_head, V, H, 0, 0});
   return v;
 }
 
 // Writes the packed copy of every layer matrix and the LM head (allocated on
-// first use) from the row-major weights, in the geometry each forward GEMM
-// call uses.
+// first use) from the row-major weights.
 static hipError_t make_packs(orion_hip_model* m) {
   const auto& d = m->desc;
   hipStream_t stream = m->dev->stream;
-  auto one = [&](uint16_t** dst, const uint16_t* w, int64_t N, int64_t K,
-                 bool deferred) -> hipError_t {
-    const size_t bytes = gemv_packed_bytes(N, K, deferred);
+  auto one = [&](const MatrixRef& r) -> hipError_t {
+    const size_t bytes = packed_weight_bytes(r.N, r.K);
     if (!bytes) return hipErrorInvalidValue;
-    if (!*dst) {
-      hipError_t e = m->alloc(dst, bytes / 2);
+    if (!*r.packed) {
+      hipError_t e = m->alloc(r.packed, bytes / 2);
       if (e != hipSuccess) return e;
     }
-    return launch_gemv_pack(stream, w, N, K, deferred, *dst);
+    return launch_pack_weights(stream, *r.rowmajor, r.N, r.K, r.pair_dim, r.pair_cols, *r.packed);
   };
   if (!m->rowmajor_live) return hipErrorInvalidValue;
   for (const MatrixRef& r : matrices(m)) {
-    hipError_t e = one(r.packed, *r.rowmajor, r.N, r.K, r.deferred);
+    hipError_t e = one(r);
     if (e != hipSuccess) return e;
   }
   if (d.tied_lm_head) {
-    hipError_t e = one(&m->p_head, m->w_embed, d.vocab_size, d.hidden_size, false);
+    hipError_t e = one({&m->w_embed, &m->p_head, d.vocab_size, d.hidden_size, 0, 0});
     if (e != hipSuccess) return e;
   }
   m->packs_valid = true;
@@ -1374,7 +1384,8 @@ static hipError_t ensure_rowmajor(orion_hip_model* m) {
   for (const MatrixRef& r : matrices(m)) {
     hipError_t e = m->alloc(r.rowmajor, (size_t)(r.N * r.K));
     if (e == hipSuccess)
-      e = launch_gemv_unpack(m->dev->stream, *r.packed, r.N, r.K, r.deferred, *r.rowmajor);
+      e = launch_unpack_weights(m->dev->stream, *r.packed, r.N, r.K, r.pair_dim, r.pair_cols,
+                                *r.rowmajor);
     if (e != hipSuccess) return e;
   }
   m->rowmajor_live = true;
@@ -1397,41 +1408,44 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   // ---- capacity ----
   const int64_t nbt = b->block_table_offsets[S];
   HIP_TRY(st, m->hidden.reserve(n * H * 4));
-  HIP_TRY(st, m->xn.reserve(n * H * 4));
+  HIP_TRY(st, m->xn.reserve(act_frag_bytes(n, H)));
   HIP_TRY(st, m->qkv.reserve(n * m->qkvd * 4));
   HIP_TRY(st, m->qrot.reserve(n * m->qd * 4));
-  HIP_TRY(st, m->attn.reserve(n * m->qd * 4));
-  HIP_TRY(st, m->act.reserve(n * F * 4));
+  HIP_TRY(st, m->attn.reserve(act_frag_bytes(n, m->qd)));
+  HIP_TRY(st, m->act.reserve(act_frag_bytes(n, F)));
   HIP_TRY(st, m->logits.reserve(S * V * 4));
   HIP_TRY(st, m->argmax.reserve(S * 8));
-  // Decode-shaped batches run the layer with the split-K GEMM fusions: each
-  // residual-add GEMM also writes the per-row sums of squares, the next GEMM
-  // applies the RMSNorm to its input, and the QKV partials go straight into
-  // RoPE + cache write.  ORION_GEMM_FUSE=0 runs the separate launches (read
-  // per call, so a test can run one batch both ways in one process).
-  const char* fuse_env = getenv("ORION_GEMM_FUSE");
-  const bool allow_fuse = !(fuse_env && fuse_env[0] == '0');
-  const bool fused = allow_fuse && gemm_splitk_fusable(n, m->qkvd, H) &&
-                     gemm_splitk_fusable(n, H, m->qd) && gemm_splitk_fusable(n, 2 * F, H) &&
-                     gemm_splitk_fusable(n, H, F);
-  const int nslots = gemm_sumsq_slots(H);
-  if (fused) HIP_TRY(st, m->sumsq.reserve(n * nslots * 8));
-  // Every GEMM reads the packed weight copies (the decode kernel's order),
-  // made on the first forward after a weight write, after which the row-major
-  // matrices are freed: one copy of each weight stays in HBM.
-  // ORION_GEMV_PACK=0 keeps the row-major matrices and reads them instead
-  // (A/B knob, read once).
+  // Every GEMM reads the packed weight copies, made on the first forward after
+  // a weight write, after which the row-major matrices are freed: one copy of
+  // each weight stays in HBM.  ORION_GEMV_PACK=0 keeps the row-major matrices
+  // and reads them instead (A/B knob, read once).
   static const bool allow_pack = [] {
     const char* v = getenv("ORION_GEMV_PACK");
     return !(v && v[0] == '0');
   }();
-  const bool pack_layers = allow_pack, pack_head = allow_pack;
   if (allow_pack) {
     if (!m->packs_valid) HIP_TRY(st, make_packs(m));
     HIP_TRY(st, release_rowmajor(m));
   } else {
     HIP_TRY(st, ensure_rowmajor(m));
   }
+  // Up to kRowsMax rows the projections run as launch_gemm_rows, which apply
+  // the RMSNorm to their input from the rows' sums of squares, and the layer
+  // fuses around them: each residual-add GEMM also writes those sums (and the
+  // next GEMM's operand), and the QKV GEMM rotates and writes the cache (heads
+  // of whole 16-column tiles).  ORION_GEMM_FUSE=0 runs these as separate
+  // launches (read per call, so a test can run one batch both ways in one
+  // process).
+  const char* fuse_env = getenv("ORION_GEMM_FUSE");
+  const bool rows_route = allow_pack && n <= kRowsMax;
+  const bool fused = rows_route && !(fuse_env && fuse_env[0] == '0');
+  const bool fused_rope = fused && m->pair_dim;
+  // activations between the layer's kernels in fragment order
+  const bool frag = rows_route && n >= kFragMinRows;
+  const bool rows_head = allow_pack && S <= kRowsMax;
+  if (rows_route || rows_head)
+    HIP_TRY(st, m->sumsq.reserve(std::min(n, kRowsMax) *
+                                 std::max(rows_sumsq_slots(H), embed_sumsq_slots(H)) * 8));
   // Attention routing, shared by every layer.  A sequence whose rows are a
   // chunk of consecutive positions with at least half a prefill tile of
   // (row, query head) pairs goes to the MFMA prefill kernel (bf16 arena);
@@ -1527,7 +1541,8 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   // ---- block ids and attention plans.  Nothing before layer 0's RoPE / KV
   // write reads the arena or the plans, so the block ids are checked and the
   // plans built on the host (and copied up) while the GPU runs the embedding
-  // and layer 0's QKV GEMM. ----
+  // and layer 0's QKV GEMM; where that GEMM writes the cache, the ids are
+  // checked before it. ----
   PrefillPlan pfp;
   DecodePlanHost plan;
   DecodePlanDev dplan, pf_merge;
@@ -1541,7 +1556,8 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   // activations decides whether the O GEMM can take them too)
   bool presplit = false;
   auto plan_attention = [&]() -> int {
-    if (int rc = validate_tables(m, b, hb)) return rc;
+    if (!fused_rope)
+      if (int rc = validate_tables(m, b, hb)) return rc;
     if (npf)
       build_prefill_order(pf_start.data(), pf_count.data(), pf_pos.data(), npf, G,
                           d.num_kv_heads, m->dev->wave_slots / 8, &pfp, d.head_dim);
@@ -1635,21 +1651,49 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   float* attn = m->attn.as<float>();
   float* act = m->act.as<float>();
 
-  double* sumsq = fused ? m->sumsq.as<double>() : nullptr;
-  // The norm a GEMM applies to its input (fused) / nothing (separate norm).
-  auto norm_in = [&](const float* weight) {
-    GemmFuse f;
-    if (fused) {
-      f.norm_sumsq = sumsq;
-      f.norm_slots = nslots;
-      f.norm_weight = weight;
-      f.norm_eps = d.rms_norm_eps;
-    }
-    return f;
+  double* sumsq = m->sumsq.as<double>();
+  uint16_t* xn_frag = frag ? m->xn.as<uint16_t>() : nullptr;
+  uint16_t* act_frag = frag ? m->act.as<uint16_t>() : nullptr;
+  // attention rows in fragment order: every row must come from the decode
+  // kernels that write it
+  const bool attn_frag = frag && !npf && decode_mfma(m->kv, Hq);
+  // A projection of the rows route: y = x W^T on packed weights.
+  auto rows_gemm = [&](const float* x, bool x_frag, const uint16_t* w, int64_t N, int64_t K,
+                       Epilogue ep, float* out) {
+    RowsGemm g;
+    g.x = x;
+    g.x_frag = x_frag;
+    g.w = w;
+    g.M = n;
+    g.N = N;
+    g.K = K;
+    g.ep = ep;
+    g.out = out;
+    return g;
   };
-  GemmFuse accumulate;  // residual-add GEMMs: out += x W^T (+ row sums of squares)
-  accumulate.sumsq_out = sumsq;
-  GemmPartials part{};
+  // ... whose input is rms_norm(hidden) * weight, from the sums of squares in
+  // `slots` slots per row.
+  auto normed = [&](RowsGemm g, const float* weight, int slots) {
+    g.norm_sumsq = sumsq;
+    g.norm_slots = slots;
+    g.norm_eps = d.rms_norm_eps;
+    if (!g.x_frag) g.norm_weight = weight;
+    return g;
+  };
+  // ... that adds to hidden and leaves what the next norm needs.
+  auto add_to_hidden = [&](RowsGemm g, const float* next_weight) -> hipError_t {
+    if (!fused) {
+      hipError_t e = gemm_rows_on(m->dev, g);
+      if (e != hipSuccess) return e;
+      return launch_norm_input(stream, hidden, nullptr, next_weight, n, H, sumsq, xn_frag, nullptr);
+    }
+    g.sumsq_out = sumsq;
+    g.out_frag = xn_frag;
+    g.next_weight = next_weight;
+    return gemm_rows_on(m->dev, g);
+  };
+  const float* normed_x = frag ? xn : hidden;
+  const int row_slots = fused ? rows_sumsq_slots(H) : embed_sumsq_slots(H);
   // Prefill-shaped batches (every layer GEMM on the LDS-tiled kernel): the
   // two RMSNorms and the SwiGLU epilogue write their outputs already split
   // into the GEMM's bf16 hi/lo operands, so the QKV, gate/up and down GEMMs
@@ -1658,35 +1702,66 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   // activations (measurement knob, read per call).
   const char* presplit_env = getenv("ORION_GEMM_PRESPLIT");
   const char* act_env = getenv("ORION_GEMM_ACT");
-  presplit = !fused && n > 64 && pack_layers && H % 8 == 0 && F % 8 == 0 &&
+  presplit = n > kRowsMax && allow_pack && H % 8 == 0 && F % 8 == 0 &&
              !(presplit_env && presplit_env[0] == '0') && !(act_env && act_env[0] == 'b');
-  // (the fused route's embed also leaves the row sums of squares, so layer
+  // (the rows route's embed also leaves the row sums of squares, so layer
   // 0's QKV GEMM applies its RMSNorm like every later layer's)
-  HIP_TRY(st, launch_embed(stream, d_tok, n, m->w_embed, H, hidden, sumsq));
+  HIP_TRY(st, launch_embed(stream, d_tok, n, m->w_embed, H, hidden, rows_route ? sumsq : nullptr,
+                           xn_frag, m->layers[0].input_norm));
+  if (fused_rope)
+    if (int rc = validate_tables(m, b, hb)) return rc;
+  const ArenaStrides as = arena_strides(m->kv);
+  int bs_log2 = 0;
+  while ((1 << bs_log2) < d.block_size) ++bs_log2;
   for (int64_t l = 0; l < d.num_layers; ++l) {
     const LayerDev& L = m->layers[l];
-    // QKV input: rms_norm(hidden) * input_norm -- inside the QKV GEMM when
-    // the embed or the previous layer's down GEMM left the sums of squares,
-    // else a kernel of its own.
-    GemmFuse qkv_f = norm_in(L.input_norm);
-    const float* qkv_x = hidden;
-    if (!qkv_f.norm_sumsq) {
+    // QKV input: rms_norm(hidden) * input_norm -- inside the QKV GEMM on the
+    // rows route, else a kernel of its own.
+    if (!rows_route)
       HIP_TRY(st, launch_rmsnorm(stream, hidden, nullptr, L.input_norm, n, H, d.rms_norm_eps, xn,
                                  presplit));
-      qkv_x = xn;
-      qkv_f.x_hilo = presplit;
+    if (rows_route) {
+      RowsGemm g = normed(rows_gemm(normed_x, frag, L.p_qkv, m->qkvd, H, Epilogue::kStore, qkv),
+                          L.input_norm, l == 0 ? embed_sumsq_slots(H) : row_slots);
+      g.bias = L.b_qkv;
+      g.pair_dim = m->pair_dim;
+      g.pair_cols = m->qd + m->kvd;
+      if (fused_rope) {
+        RopeOut& r = g.rope;
+        r.q_out = qrot;
+        r.kv_bf16 = m->kv.dtype_bf16;
+        r.kv = static_cast<char*>(m->arena) + l * as.layer * (r.kv_bf16 ? 2 : 4);
+        r.hq = (int)Hq;
+        r.hkv = d.num_kv_heads;
+        r.bs_log2 = bs_log2;
+        r.blk = as.blk;
+        r.v_off = as.v_off;
+        r.slot = as.slot;
+        r.head = as.head;
+        r.positions = d_pos;
+        r.row_seq = d_rs;
+        r.bt_off = d_btoff;
+        r.bt_ids = d_btids;
+        r.cos = m->rope_cos;
+        r.sin = m->rope_sin;
+      }
+      HIP_TRY(st, gemm_rows_on(m->dev, g));
+    } else {
+      GemmFuse f;
+      f.x_hilo = presplit;
+      if (allow_pack) f.w_packed = L.p_qkv, f.pair_dim = m->pair_dim, f.pair_cols = m->qd + m->kvd;
+      HIP_TRY(st, gemm_on(m->dev, xn, L.w_qkv, L.b_qkv, n, m->qkvd, H, Epilogue::kStore, qkv, &f));
     }
-    qkv_f.defer = &part;
-    if (pack_layers) qkv_f.w_packed = L.p_qkv, qkv_f.w_packed_deferred = true;
-    HIP_TRY(st, gemm_on(m->dev, qkv_x, L.w_qkv, L.b_qkv, n, m->qkvd, H, Epilogue::kStore, qkv,
-                        &qkv_f));
     if (l == 0)
       if (int rc = plan_attention()) return rc;
-    HIP_TRY(st, launch_rope_and_cache(stream, m->kv, m->arena, l, n, Hq, qkv, m->qkvd, qrot,
-                                      qkv + m->qd, m->qkvd, qkv + m->qd + m->kvd, m->qkvd, d_pos,
-                                      d_rs, d_btoff, d_btids, m->rope_cos, m->rope_sin, &part));
+    if (!fused_rope)
+      HIP_TRY(st, launch_rope_and_cache(stream, m->kv, m->arena, l, n, Hq, qkv, m->qkvd, qrot,
+                                        qkv + m->qd, m->qkvd, qkv + m->qd + m->kvd, m->qkvd, d_pos,
+                                        d_rs, d_btoff, d_btids, m->rope_cos, m->rope_sin));
+    AttnOut attn_out{attn};
+    if (attn_frag) attn_out.frag = m->attn.as<uint16_t>(), attn_out.mtiles = act_tiles(n);
     HIP_TRY(st, launch_paged_decode(stream, m->kv, m->arena, l, qrot, n, Hq, d_pos, d_rs, d_btoff,
-                                    d_btids, dplan, attn));
+                                    d_btids, dplan, attn_out));
     if (npf) {
       HIP_TRY(st, launch_paged_prefill(stream, m->kv, m->arena, l, qrot, Hq, d_pforder,
                                        (int64_t)pfp.order.size(), d_pfstart, d_pfcount, d_pfpos,
@@ -1694,40 +1769,60 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
       if (pf_split)
         HIP_TRY(st, launch_split_merge(stream, d.head_dim, n, Hq, pf_merge, attn));
     }
-    GemmFuse o_f = accumulate;
+    const float* next_norm = l + 1 < d.num_layers ? m->layers[l + 1].input_norm : m->final_norm;
+    if (rows_route) {
+      HIP_TRY(st, add_to_hidden(rows_gemm(attn, attn_frag, L.p_o, H, m->qd, Epilogue::kAccumulate,
+                                          hidden), L.post_norm));
+      RowsGemm gu = normed(rows_gemm(normed_x, frag, L.p_gu, 2 * F, H, Epilogue::kSwiGLU, act),
+                           L.post_norm, row_slots);
+      gu.out_frag = act_frag;
+      HIP_TRY(st, gemm_rows_on(m->dev, gu));
+      HIP_TRY(st, add_to_hidden(rows_gemm(act, frag, L.p_down, H, F, Epilogue::kAccumulate,
+                                          hidden), next_norm));
+      continue;
+    }
+    GemmFuse o_f;
     o_f.x_hilo = o_presplit;
-    if (pack_layers) o_f.w_packed = L.p_o;
+    if (allow_pack) o_f.w_packed = L.p_o;
     HIP_TRY(st, gemm_on(m->dev, attn, L.w_o, nullptr, n, H, m->qd, Epilogue::kAccumulate,
                         hidden, &o_f));
-    GemmFuse gu_f = norm_in(L.post_norm);
-    if (pack_layers) gu_f.w_packed = L.p_gu;
-    if (!fused)
-      HIP_TRY(st, launch_rmsnorm(stream, hidden, nullptr, L.post_norm, n, H, d.rms_norm_eps, xn,
-                                 presplit));
+    HIP_TRY(st, launch_rmsnorm(stream, hidden, nullptr, L.post_norm, n, H, d.rms_norm_eps, xn,
+                               presplit));
+    GemmFuse gu_f;
+    if (allow_pack) gu_f.w_packed = L.p_gu;
     gu_f.x_hilo = gu_f.out_hilo = presplit;
-    HIP_TRY(st, gemm_on(m->dev, fused ? hidden : xn, L.w_gu, nullptr, n, 2 * F, H,
-                        Epilogue::kSwiGLU, act, &gu_f));
-    GemmFuse down_f = accumulate;
+    HIP_TRY(st, gemm_on(m->dev, xn, L.w_gu, nullptr, n, 2 * F, H, Epilogue::kSwiGLU, act, &gu_f));
+    GemmFuse down_f;
     down_f.x_hilo = presplit;
-    if (pack_layers) down_f.w_packed = L.p_down;
+    if (allow_pack) down_f.w_packed = L.p_down;
     HIP_TRY(st, gemm_on(m->dev, act, L.w_down, nullptr, n, H, F, Epilogue::kAccumulate, hidden,
                         &down_f));
   }
   // Final norm on the last row of each sequence only (norm is row-wise, so
   // this equals norming all rows and then gathering), then the LM head.
-  // When every row is its sequence's last row (a decode batch) and the layer
-  // GEMMs left the row sums of squares, the LM head applies the norm while
-  // staging its input, as the layer GEMMs do.
-  bool head_norm = fused && S == n && gemm_splitk_fusable(S, V, H);
-  for (int64_t i = 0; head_norm && i < S; ++i) head_norm = hb.last_rows[i] == (int32_t)i;
-  GemmFuse head_f = head_norm ? norm_in(m->final_norm) : GemmFuse{};
-  if (!head_norm)
-    HIP_TRY(st, launch_rmsnorm(stream, hidden, d_last, m->final_norm, S, H, d.rms_norm_eps, xn));
-  const uint16_t* head = m->w_lm ? m->w_lm : m->w_embed;
+  // When every row is its sequence's last row (a decode batch) on the rows
+  // route, the last down projection left the LM head's input.
+  bool head_ready = rows_route && S == n;
+  for (int64_t i = 0; head_ready && i < S; ++i) head_ready = hb.last_rows[i] == (int32_t)i;
   float* logits = m->logits.as<float>();
-  if (pack_head) head_f.w_packed = m->p_head;
-  HIP_TRY(st, gemm_on(m->dev, head_norm ? hidden : xn, head, nullptr, S, V, H, Epilogue::kStore,
-                      logits, &head_f));
+  if (rows_head) {
+    const bool head_frag = S >= kFragMinRows;
+    if (!head_ready)
+      HIP_TRY(st, launch_norm_input(stream, hidden, d_last, m->final_norm, S, H, sumsq,
+                                    head_frag ? m->xn.as<uint16_t>() : nullptr,
+                                    head_frag ? nullptr : xn));
+    RowsGemm g = normed(rows_gemm(head_frag || !head_ready ? xn : hidden, head_frag, m->p_head, V,
+                                  H, Epilogue::kStore, logits),
+                        m->final_norm, head_ready ? row_slots : embed_sumsq_slots(H));
+    g.M = S;
+    HIP_TRY(st, gemm_rows_on(m->dev, g));
+  } else {
+    GemmFuse f;
+    if (allow_pack) f.w_packed = m->p_head;
+    HIP_TRY(st, launch_rmsnorm(stream, hidden, d_last, m->final_norm, S, H, d.rms_norm_eps, xn));
+    HIP_TRY(st, gemm_on(m->dev, xn, m->w_lm ? m->w_lm : m->w_embed, nullptr, S, V, H,
+                        Epilogue::kStore, logits, &f));
+  }
   m->last_rows = S;
   if (argmax_out) {
     HIP_TRY(st, launch_argmax(stream, logits, S, V, m->argmax.as<int64_t>()));
@@ -1861,21 +1956,21 @@ ORION_EXPORT int orion_hip_paged_attention_decode(
   HIP_TRY(st, hipSetDevice(dev->ordinal));
   if (!dev->ktiming) {
     HIP_TRY(st, launch_paged_decode(dev->stream, g, d_arena, layer, d_q, num_rows, num_q_heads,
-                                    d_positions, d_row_seq, d_bt_offsets, d_bt_ids, plan->view(g.dtype_bf16),
-                                    d_out));
+                                    d_positions, d_row_seq, d_bt_offsets, d_bt_ids,
+                                    plan->view(g.dtype_bf16), AttnOut{d_out}));
     return ORION_HIP_OK;
   }
   // Timed: the split-K kernel and the merge kernel as separate launches.
   DecodePlanDev pv = plan->view(g.dtype_bf16);
   HIP_TRY(st, timed_launch(dev, 0, [&] {
             return launch_paged_decode(dev->stream, g, d_arena, layer, d_q, num_rows, num_q_heads,
-                                       d_positions, d_row_seq, d_bt_offsets, d_bt_ids, pv, d_out,
-                                       DecodePhase::kSplit);
+                                       d_positions, d_row_seq, d_bt_offsets, d_bt_ids, pv,
+                                       AttnOut{d_out}, DecodePhase::kSplit);
           }));
   HIP_TRY(st, timed_launch(dev, 1, [&] {
             return launch_paged_decode(dev->stream, g, d_arena, layer, d_q, num_rows, num_q_heads,
-                                       d_positions, d_row_seq, d_bt_offsets, d_bt_ids, pv, d_out,
-                                       DecodePhase::kMerge);
+                                       d_positions, d_row_seq, d_bt_offsets, d_bt_ids, pv,
+                                       AttnOut{d_out}, DecodePhase::kMerge);
           }));
   return ORION_HIP_OK;
 }
