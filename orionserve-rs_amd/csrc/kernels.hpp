@@ -343,12 +343,10 @@ struct SampleParams {
   float repetition_penalty;
 };
 constexpr int64_t kSampleMaxVocab = 262144;
-// logits [rows, vocab] are filtered in place; probs_ws holds rows * vocab
-// floats; out gets one token per row.
+// logits [rows, vocab] are filtered in place; out gets one token per row.
 hipError_t launch_sample(hipStream_t st, float* logits, int64_t rows, int64_t vocab,
                          const SampleParams* params, const int64_t* prev_off,
-                         const uint32_t* prev_tok, const float* uniform, float* probs_ws,
-                         int32_t* out);
+                         const uint32_t* prev_tok, const float* uniform, int32_t* out);
 
 // ---- elementwise / normalisation -------------------------------------------
 // sumsq: when set, also the row sums of squares, one f64 per 64 columns

@@ -148,7 +148,7 @@ struct orion_hip_device {
   DevBuf gemm_ws;
   DevBuf prefill_order;  // op-level prefill work list (+ key-part merge lists)
   DevBuf prefill_ws;     // op-level prefill key-part partials
-  DevBuf sample_io, sample_ws;  // sampler inputs/outputs and probabilities
+  DevBuf sample_io;  // sampler inputs and outputs
   // This device's address of the file-scope `scratch` array
   // (orion_hip_gemm_noalloc); never freed.
   void* noalloc_scratch = nullptr;
@@ -395,7 +395,6 @@ ORION_EXPORT void orion_hip_device_close(orion_hip_device* dev) {
   dev->prefill_order.release();
   dev->prefill_ws.release();
   dev->sample_io.release();
-  dev->sample_ws.release();
   (void)hipStreamDestroy(dev->stream);
   delete dev;
 }
@@ -1007,7 +1006,6 @@ int sample_on(orion_hip_device* dev, float* d_logits, int64_t rows, int64_t voca
   std::memcpy(host.data() + o_uni, uniform, rows * 4);
   HIP_TRY(st, hipSetDevice(dev->ordinal));
   HIP_TRY(st, dev->sample_io.reserve(total));
-  HIP_TRY(st, dev->sample_ws.reserve((size_t)rows * vocab * 4));
   hipStream_t stream = dev->stream;
   char* d = static_cast<char*>(dev->sample_io.ptr);
   HIP_TRY(st, hipMemcpyAsync(d, host.data(), o_out, hipMemcpyHostToDevice, stream));
@@ -1016,7 +1014,7 @@ int sample_on(orion_hip_device* dev, float* d_logits, int64_t rows, int64_t voca
                             reinterpret_cast<const int64_t*>(d + o_off),
                             reinterpret_cast<const uint32_t*>(d + o_tok),
                             reinterpret_cast<const float*>(d + o_uni),
-                            dev->sample_ws.as<float>(), reinterpret_cast<int32_t*>(d + o_out)));
+                            reinterpret_cast<int32_t*>(d + o_out)));
   HIP_TRY(st, hipMemcpyAsync(tokens, d + o_out, rows * 4, hipMemcpyDeviceToHost, stream));
   HIP_TRY(st, hipStreamSynchronize(stream));
   for (int64_t r = 0; r < rows; ++r)  // a greedy row with no number above -inf
