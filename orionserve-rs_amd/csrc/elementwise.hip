@@ -455,6 +455,27 @@ hipError_t launch_argmax(hipStream_t st, const float* logits, int64_t rows, int6
   return hipGetLastError();
 }
 
+// Small transfers between pinned host memory and the device as a kernel: one
+// 16-byte word per thread over the link.  In stream order with the kernels
+// around it, where a copy command hands the stream to a DMA engine and back
+// (184 KB of logits: 27 us between the last kernel and the copy's
+// start, 32 us from its end to the caller).
+__global__ void __launch_bounds__(256)
+    host_copy_kernel(const uint4* __restrict__ src, int64_t words, uint4* __restrict__ dst) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < words) dst[i] = src[i];
+}
+
+hipError_t launch_host_copy(hipStream_t st, void* dst, const void* src, size_t bytes) {
+  if (bytes == 0) return hipSuccess;
+  if ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15)
+    return hipErrorInvalidValue;
+  const int64_t words = (int64_t)((bytes + 15) / 16);
+  hipLaunchKernelGGL(host_copy_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st,
+                     static_cast<const uint4*>(src), words, static_cast<uint4*>(dst));
+  return hipGetLastError();
+}
+
 __global__ void f32_to_bf16_kernel(const float* __restrict__ in, uint16_t* __restrict__ out,
                                    int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;

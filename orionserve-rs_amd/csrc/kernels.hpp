@@ -379,6 +379,11 @@ hipError_t launch_rope_and_cache(hipStream_t st, const KvGeom& kv, void* arena, 
 hipError_t launch_silu_mul(hipStream_t st, float* gate, const float* up, int64_t count);
 hipError_t launch_argmax(hipStream_t st, const float* logits, int64_t rows, int64_t cols,
                          int64_t* out);
+// Copies between pinned host memory and the device in 16-byte words (both ends
+// 16-byte aligned and allocated to a multiple of 16 bytes), for transfers of up
+// to kHostCopyMax bytes; larger ones are a copy command's.
+constexpr size_t kHostCopyMax = size_t(1) << 20;
+hipError_t launch_host_copy(hipStream_t st, void* dst, const void* src, size_t bytes);
 hipError_t launch_f32_to_bf16(hipStream_t st, const float* in, uint16_t* out, int64_t count);
 hipError_t launch_synthetic_bf16(hipStream_t st, uint16_t* out, int64_t count, uint64_t key,
                                  float mul);

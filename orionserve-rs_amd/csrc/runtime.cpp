@@ -93,6 +93,36 @@ struct DevBuf {
   }
 };
 
+// Pinned host memory that grows on demand; the caller has waited for the work
+// that uses it before it grows or is released.
+struct PinnedBuf {
+  void* ptr = nullptr;
+  size_t bytes = 0;
+  hipError_t reserve(size_t want) {
+    if (want <= bytes) return hipSuccess;
+    release();
+    const size_t cap = (std::max<size_t>(want * 2, 1 << 16) + 15) & ~(size_t)15;
+    hipError_t e = hipHostMalloc(&ptr, cap, hipHostMallocDefault);
+    if (e != hipSuccess) {
+      ptr = nullptr;
+      return e;
+    }
+    bytes = cap;
+    return hipSuccess;
+  }
+  void release() {
+    if (ptr) (void)hipHostFree(ptr);
+    ptr = nullptr;
+    bytes = 0;
+  }
+};
+
+// Pinned memory to the device, in stream order.
+hipError_t upload(hipStream_t st, void* dst, const void* pinned, size_t bytes) {
+  if (bytes <= kHostCopyMax) return launch_host_copy(st, dst, pinned, bytes);
+  return hipMemcpyAsync(dst, pinned, bytes, hipMemcpyHostToDevice, st);
+}
+
 uint16_t host_f32_to_bf16(float f) {
   uint32_t u;
   std::memcpy(&u, &f, 4);
@@ -148,7 +178,8 @@ struct orion_hip_device {
   DevBuf gemm_ws;
   DevBuf prefill_order;  // op-level prefill work list (+ key-part merge lists)
   DevBuf prefill_ws;     // op-level prefill key-part partials
-  DevBuf sample_io;  // sampler inputs and outputs
+  DevBuf sample_io;      // sampler inputs
+  PinnedBuf sample_host; // their staging, and the sampled tokens
   // This device's address of the file-scope `scratch` array
   // (orion_hip_gemm_noalloc); never freed.
   void* noalloc_scratch = nullptr;
@@ -255,18 +286,17 @@ struct orion_hip_model {
   int64_t last_rows = 0;  // rows of `logits` the last forward produced
 
   // activations / batch buffers (grown on demand)
-  DevBuf hidden, xn, qkv, qrot, attn, act, logits, argmax, ws, sumsq;
+  DevBuf hidden, xn, qkv, qrot, attn, act, logits, ws, sumsq;
   DevBuf b_batch, b_plan;  // the batch and the attention plans (one copy each)
-  void* pinned[2] = {nullptr, nullptr};  // their pinned staging areas
-  size_t pinned_bytes[2] = {0, 0};
+  PinnedBuf h_batch, h_plan;  // their staging areas
+  PinnedBuf h_out;            // logits and greedy tokens on their way out
 
   ~orion_hip_model() {
     for (void* p : allocations) (void)hipFree(p);
-    for (DevBuf* b : {&hidden, &xn, &qkv, &qrot, &attn, &act, &logits, &argmax, &ws, &sumsq,
+    for (DevBuf* b : {&hidden, &xn, &qkv, &qrot, &attn, &act, &logits, &ws, &sumsq,
                       &b_batch, &b_plan})
       b->release();
-    for (void* p : pinned)
-      if (p) (void)hipHostFree(p);
+    for (PinnedBuf* b : {&h_batch, &h_plan, &h_out}) b->release();
   }
 
   // Frees one allocation made by alloc (the device is synchronised first).
@@ -395,6 +425,7 @@ ORION_EXPORT void orion_hip_device_close(orion_hip_device* dev) {
   dev->prefill_order.release();
   dev->prefill_ws.release();
   dev->sample_io.release();
+  dev->sample_host.release();
   (void)hipStreamDestroy(dev->stream);
   delete dev;
 }
@@ -988,35 +1019,38 @@ int sample_on(orion_hip_device* dev, float* d_logits, int64_t rows, int64_t voca
   if (prev_off[0] != 0) return internal(st, "prev_offsets[0] must be 0");
   const int64_t nprev = prev_off[rows];
   if (nprev > 0 && !prev_tok) return internal(st, "null prev_tokens");
-  // One staging copy: params | offsets | tokens | uniforms | outputs.
+  // One staging area: params | offsets | tokens | uniforms, copied up, and the
+  // outputs, which the kernel writes there.  (Each call ends with a stream
+  // sync, so the area is free.)
   const size_t o_par = 0;
   const size_t o_off = (o_par + rows * sizeof(SampleParams) + 7) & ~(size_t)7;
   const size_t o_tok = o_off + (rows + 1) * 8;
   const size_t o_uni = (o_tok + nprev * 4 + 3) & ~(size_t)3;
-  const size_t o_out = o_uni + rows * 4;
+  const size_t o_out = (o_uni + rows * 4 + 15) & ~(size_t)15;
   const size_t total = o_out + rows * 4;
-  std::vector<char> host(total);
+  HIP_TRY(st, hipSetDevice(dev->ordinal));
+  HIP_TRY(st, dev->sample_host.reserve(total));
+  HIP_TRY(st, dev->sample_io.reserve(o_out));
+  char* host = static_cast<char*>(dev->sample_host.ptr);
   for (int64_t r = 0; r < rows; ++r) {
     const SampleParams sp{params[r].temperature, params[r].top_k, params[r].top_p,
                           params[r].repetition_penalty};
-    std::memcpy(host.data() + o_par + r * sizeof(SampleParams), &sp, sizeof(sp));
+    std::memcpy(host + o_par + r * sizeof(SampleParams), &sp, sizeof(sp));
   }
-  std::memcpy(host.data() + o_off, prev_off, (rows + 1) * 8);
-  if (nprev) std::memcpy(host.data() + o_tok, prev_tok, nprev * 4);
-  std::memcpy(host.data() + o_uni, uniform, rows * 4);
-  HIP_TRY(st, hipSetDevice(dev->ordinal));
-  HIP_TRY(st, dev->sample_io.reserve(total));
+  std::memcpy(host + o_off, prev_off, (rows + 1) * 8);
+  if (nprev) std::memcpy(host + o_tok, prev_tok, nprev * 4);
+  std::memcpy(host + o_uni, uniform, rows * 4);
   hipStream_t stream = dev->stream;
   char* d = static_cast<char*>(dev->sample_io.ptr);
-  HIP_TRY(st, hipMemcpyAsync(d, host.data(), o_out, hipMemcpyHostToDevice, stream));
+  HIP_TRY(st, upload(stream, d, host, o_out));
   HIP_TRY(st, launch_sample(stream, d_logits, rows, vocab,
                             reinterpret_cast<const SampleParams*>(d + o_par),
                             reinterpret_cast<const int64_t*>(d + o_off),
                             reinterpret_cast<const uint32_t*>(d + o_tok),
                             reinterpret_cast<const float*>(d + o_uni),
-                            reinterpret_cast<int32_t*>(d + o_out)));
-  HIP_TRY(st, hipMemcpyAsync(tokens, d + o_out, rows * 4, hipMemcpyDeviceToHost, stream));
+                            reinterpret_cast<int32_t*>(host + o_out)));
   HIP_TRY(st, hipStreamSynchronize(stream));
+  std::memcpy(tokens, host + o_out, rows * 4);
   for (int64_t r = 0; r < rows; ++r)  // a greedy row with no number above -inf
     if (tokens[r] < 0) return internal(st, "row %lld: argmax over empty logits", (long long)r);
   return ORION_HIP_OK;
@@ -1412,7 +1446,6 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   HIP_TRY(st, m->attn.reserve(act_frag_bytes(n, m->qd)));
   HIP_TRY(st, m->act.reserve(act_frag_bytes(n, F)));
   HIP_TRY(st, m->logits.reserve(S * V * 4));
-  HIP_TRY(st, m->argmax.reserve(S * 8));
   // Every GEMM reads the packed weight copies, made on the first forward after
   // a weight write, after which the row-major matrices are freed: one copy of
   // each weight stays in HBM.  ORION_GEMV_PACK=0 keeps the row-major matrices
@@ -1485,27 +1518,8 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   }
   const int64_t npf = (int64_t)pf_start.size();
 
-  // Pinned staging area i (0: the batch, 1: the attention plans), grown on
-  // demand.  Each forward ends with a stream sync, so the previous forward's
-  // copies out of both are complete.
-  auto staging = [&](int i, size_t bytes) -> hipError_t {
-    if (bytes <= m->pinned_bytes[i]) return hipSuccess;
-    if (m->pinned[i]) {
-      hipError_t e = hipStreamSynchronize(stream);
-      if (e == hipSuccess) e = hipHostFree(m->pinned[i]);
-      if (e != hipSuccess) return e;
-      m->pinned[i] = nullptr;
-      m->pinned_bytes[i] = 0;
-    }
-    const size_t cap = std::max<size_t>(bytes * 2, 1 << 16);
-    hipError_t e = hipHostMalloc(&m->pinned[i], cap, hipHostMallocDefault);
-    if (e != hipSuccess) {
-      m->pinned[i] = nullptr;
-      return e;
-    }
-    m->pinned_bytes[i] = cap;
-    return hipSuccess;
-  };
+  // (Each forward ends with a stream sync, so the previous forward's use of
+  // the staging areas is complete.)
 
   // ---- upload the batch: tokens, positions, row sequences, last rows and
   // block tables, one pinned staging area, one copy ----
@@ -1516,17 +1530,17 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   const size_t o_btoff = (o_last + S * 4 + 7) & ~(size_t)7;
   const size_t o_btids = o_btoff + (S + 1) * 8;
   const size_t total = o_btids + nbt * 4;
-  HIP_TRY(st, staging(0, total));
+  HIP_TRY(st, m->h_batch.reserve(total));
   HIP_TRY(st, m->b_batch.reserve(total));
   {
-    char* hp = static_cast<char*>(m->pinned[0]);
+    char* hp = static_cast<char*>(m->h_batch.ptr);
     std::memcpy(hp + o_tok, b->tokens, n * 4);
     std::memcpy(hp + o_pos, b->positions, n * 4);
     std::memcpy(hp + o_rs, hb.row_seq.data(), n * 4);
     std::memcpy(hp + o_last, hb.last_rows.data(), S * 4);
     std::memcpy(hp + o_btoff, b->block_table_offsets, (S + 1) * 8);
     std::memcpy(hp + o_btids, b->block_table_ids, nbt * 4);
-    HIP_TRY(st, hipMemcpyAsync(m->b_batch.ptr, hp, total, hipMemcpyHostToDevice, stream));
+    HIP_TRY(st, upload(stream, m->b_batch.ptr, hp, total));
   }
   const char* dp = m->b_batch.as<char>();
   const uint32_t* d_tok = reinterpret_cast<const uint32_t*>(dp + o_tok);
@@ -1582,9 +1596,9 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
     const size_t o_pfparts = o_pfsplit + (pf_split ? pfp.split_rows.size() * 4 : 0);
     const size_t o_packrows = o_pfparts + (pf_split ? pfp.row_parts.size() * 4 : 0);
     const size_t ptotal = std::max<size_t>(o_packrows + plan.pack_rows.size() * 4, 8);
-    HIP_TRY(st, staging(1, ptotal));
+    HIP_TRY(st, m->h_plan.reserve(ptotal));
     HIP_TRY(st, m->b_plan.reserve(ptotal));
-    char* hp = static_cast<char*>(m->pinned[1]);
+    char* hp = static_cast<char*>(m->h_plan.ptr);
     std::memcpy(hp + o_work, plan.work.data(), plan.work.size() * sizeof(DecodeWork));
     std::memcpy(hp + o_nsplit, plan.row_nsplit.data(), plan.row_nsplit.size() * 4);
     std::memcpy(hp + o_pfoff, pf_btoff.data(), npf * 8);
@@ -1599,7 +1613,7 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
     }
     std::memcpy(hp + o_packrows, plan.pack_rows.data(), plan.pack_rows.size() * 4);
     char* pp = m->b_plan.as<char>();
-    HIP_TRY(st, hipMemcpyAsync(pp, hp, ptotal, hipMemcpyHostToDevice, stream));
+    HIP_TRY(st, upload(stream, pp, hp, ptotal));
     dplan.work = reinterpret_cast<const DecodeWork*>(pp + o_work);
     dplan.row_nsplit = reinterpret_cast<const int32_t*>(pp + o_nsplit);
     dplan.num_work = (int)plan.work.size();
@@ -1706,8 +1720,14 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   // 0's QKV GEMM applies its RMSNorm like every later layer's)
   HIP_TRY(st, launch_embed(stream, d_tok, n, m->w_embed, H, hidden, rows_route ? sumsq : nullptr,
                            xn_frag, m->layers[0].input_norm));
+  // (a refused batch waits for what it has queued: the staging areas are free
+  // again when the call returns)
+  auto refused = [&](int rc) {
+    (void)hipStreamSynchronize(stream);
+    return rc;
+  };
   if (fused_rope)
-    if (int rc = validate_tables(m, b, hb)) return rc;
+    if (int rc = validate_tables(m, b, hb)) return refused(rc);
   const ArenaStrides as = arena_strides(m->kv);
   int bs_log2 = 0;
   while ((1 << bs_log2) < d.block_size) ++bs_log2;
@@ -1751,7 +1771,7 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
       HIP_TRY(st, gemm_on(m->dev, xn, L.w_qkv, L.b_qkv, n, m->qkvd, H, Epilogue::kStore, qkv, &f));
     }
     if (l == 0)
-      if (int rc = plan_attention()) return rc;
+      if (int rc = plan_attention()) return refused(rc);
     if (!fused_rope)
       HIP_TRY(st, launch_rope_and_cache(stream, m->kv, m->arena, l, n, Hq, qkv, m->qkvd, qrot,
                                         qkv + m->qd, m->qkvd, qkv + m->qd + m->kvd, m->qkvd, d_pos,
@@ -1822,13 +1842,22 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
                         Epilogue::kStore, logits, &f));
   }
   m->last_rows = S;
-  if (argmax_out) {
-    HIP_TRY(st, launch_argmax(stream, logits, S, V, m->argmax.as<int64_t>()));
-    HIP_TRY(st, hipMemcpyAsync(argmax_out, m->argmax.ptr, S * 8, hipMemcpyDeviceToHost, stream));
-  }
-  if (logits_out)
-    HIP_TRY(st, hipMemcpyAsync(logits_out, logits, S * V * 4, hipMemcpyDeviceToHost, stream));
+  // Small outputs leave through pinned memory: the greedy tokens written there
+  // by their kernel, the logits copied by one.
+  const size_t logit_bytes = (size_t)(S * V) * 4, o_logits = (size_t)(S * 8 + 15) & ~(size_t)15;
+  const bool logits_pinned = logits_out && logit_bytes <= kHostCopyMax;
+  if (argmax_out || logits_pinned)
+    HIP_TRY(st, m->h_out.reserve(o_logits + (logits_pinned ? logit_bytes : 0)));
+  char* h_out = static_cast<char*>(m->h_out.ptr);
+  if (argmax_out)
+    HIP_TRY(st, launch_argmax(stream, logits, S, V, reinterpret_cast<int64_t*>(h_out)));
+  if (logits_pinned)
+    HIP_TRY(st, launch_host_copy(stream, h_out + o_logits, logits, logit_bytes));
+  else if (logits_out)
+    HIP_TRY(st, hipMemcpyAsync(logits_out, logits, logit_bytes, hipMemcpyDeviceToHost, stream));
   HIP_TRY(st, hipStreamSynchronize(stream));
+  if (argmax_out) std::memcpy(argmax_out, h_out, S * 8);
+  if (logits_pinned) std::memcpy(logits_out, h_out + o_logits, logit_bytes);
   return ORION_HIP_OK;
 }
 
