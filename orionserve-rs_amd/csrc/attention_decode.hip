@@ -63,13 +63,19 @@ struct KvVec<uint16_t> {
   }
 };
 
-template <typename T, int D, int G>
+// Partial results of a wave whose row the workgroup merges (GROUP): G x D
+// unnormalised outputs, then (max, sum) per head, in LDS.
+template <int D, int G>
+constexpr int group_part_floats() { return G * D + 2 * G; }
+
+template <typename T, int D, int G, bool GROUP = false>
 __device__ __forceinline__ void decode_wave_valu(
     const T* __restrict__ kv_layer, int64_t blk_stride, int64_t v_off, int64_t slot_stride,
     int64_t head_stride, int bs_log2, int num_q_heads, const float* __restrict__ q,
     const uint32_t* __restrict__ tbl,
     int max_splits, float scale, float* __restrict__ out, float* __restrict__ ws_o,
-    float* __restrict__ ws_ml, int row, int kvh, int start, int end, int split, int nsplit) {
+    float* __restrict__ ws_ml, int row, int kvh, int start, int end, int split, int nsplit,
+    float* part = nullptr) {
   constexpr int EPL = KvVec<T>::EPL;
   constexpr int CH = D / EPL;   // lanes per token vector
   constexpr int TPW = 64 / CH;  // tokens per wave load
@@ -81,6 +87,12 @@ __device__ __forceinline__ void decode_wave_valu(
   const int t = lane / CH;  // token slot within a wave load
   const int c = lane % CH;  // chunk of the head vector
   const int bs_mask = (1 << bs_log2) - 1;
+
+  // Block-table slice of this chunk (tbl points at its first entry), one
+  // entry per lane.
+  const int first_blk = start >> bs_log2;
+  const int nblk = ((end - 1) >> bs_log2) - first_blk + 1;
+  const int my_blk = lane < nblk ? (int)tbl[lane] : 0;
 
   // Query chunk for all G heads of the group.
   float qr[G][EPL];
@@ -99,12 +111,6 @@ __device__ __forceinline__ void decode_wave_valu(
     }
   }
 
-  // Block-table slice of this chunk (tbl points at its first entry), one
-  // entry per lane.
-  const int first_blk = start >> bs_log2;
-  const int nblk = ((end - 1) >> bs_log2) - first_blk + 1;
-  const int my_blk = lane < nblk ? (int)tbl[lane] : 0;
-
   const T* kbase = kv_layer + (int64_t)kvh * head_stride + c * EPL;
 
   float m[G], l[G], o[G][EPL];
@@ -116,19 +122,22 @@ __device__ __forceinline__ void decode_wave_valu(
     for (int e = 0; e < EPL; ++e) o[g][e] = 0.f;
   }
 
-  for (int base = start; base < end; base += 16) {
-    float kf[R][EPL], vf[R][EPL];
-    bool valid[R];
+  auto load = [&](int base, float (&kf)[R][EPL], float (&vf)[R][EPL]) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int j = base + r * TPW + t;
-      valid[r] = j < end;
-      const int bi = valid[r] ? (j >> bs_log2) - first_blk : 0;
+      const bool valid = j < end;
+      const int bi = valid ? (j >> bs_log2) - first_blk : 0;
       const int blk = __shfl(my_blk, bi);
       const int64_t off = (int64_t)blk * blk_stride + (int64_t)(j & bs_mask) * slot_stride;
-      KvVec<T>::load(kbase + off, valid[r], kf[r]);
-      KvVec<T>::load(kbase + off + v_off, valid[r], vf[r]);
+      KvVec<T>::load(kbase + off, valid, kf[r]);
+      KvVec<T>::load(kbase + off + v_off, valid, vf[r]);
     }
+  };
+  auto compute = [&](int base, const float (&kf)[R][EPL], const float (&vf)[R][EPL]) {
+    bool valid[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) valid[r] = base + r * TPW + t < end;
     // Partial dot products over this lane's chunk, then sum over the CH lanes.
     float s[R][G];
 #pragma unroll
@@ -170,7 +179,22 @@ __device__ __forceinline__ void decode_wave_valu(
         o[g][e] = acc;
       }
     }
+  };
+  if constexpr (GROUP) {
+    // the (at most two) steps of a grouped piece, both in flight
+    float k0[R][EPL], v0[R][EPL], k1[R][EPL], v1[R][EPL];
+    load(start, k0, v0);
+    if (start + 16 < end) load(start + 16, k1, v1);
+    compute(start, k0, v0);
+    if (start + 16 < end) compute(start + 16, k1, v1);
+  } else {
+    for (int base = start; base < end; base += 16) {
+      float kf[R][EPL], vf[R][EPL];
+      load(base, kf, vf);
+      compute(base, kf, vf);
+    }
   }
+
 
   // Merge the TPW token groups (lanes c, c+CH, c+2CH, ...).
 #pragma unroll
@@ -195,7 +219,17 @@ __device__ __forceinline__ void decode_wave_valu(
 
   if (t != 0) return;
   const int64_t head0 = (int64_t)row * num_q_heads + (int64_t)kvh * G;
-  if (nsplit == 1) {
+  if constexpr (GROUP) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+#pragma unroll
+      for (int e = 0; e < EPL; e += 4)
+        *reinterpret_cast<float4*>(part + g * D + c * EPL + e) =
+            make_float4(o[g][e], o[g][e + 1], o[g][e + 2], o[g][e + 3]);
+      if (c == 0)
+        *reinterpret_cast<float2*>(part + G * D + 2 * g) = make_float2(m[g], l[g]);
+    }
+  } else if (nsplit == 1) {
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       const float inv = 1.f / l[g];
@@ -273,14 +307,15 @@ __device__ __forceinline__ uint4 kv_load16(const uint16_t* p) {
 // PR > 1: a packed item -- the query columns hold the G heads of each of up
 // to PR rows (prow[0 .. PR), -1 unused) that share this piece's blocks;
 // column c is head c % G of row prow[c / G].
-template <int D, int G, bool STREAM, bool BIG_BLOCKS, int PR = 1>
+template <int D, int G, bool STREAM, bool BIG_BLOCKS, int PR = 1, bool GROUP = false>
 __device__ __forceinline__ void decode_wave_mfma2(
     const uint16_t* __restrict__ kv_layer, uint32_t blk_stride, uint32_t v_off,
     uint32_t slot_stride, uint32_t head_stride, int bs_log2, int num_q_heads, const float* __restrict__ q,
     const uint32_t* __restrict__ tbl, int blk0, int max_splits, float scale,
     const AttnOut& out, float* __restrict__ ws_o, float* __restrict__ ws_ml, uint16_t* VL,
     uint16_t* QL, uint16_t* KL, int row, int kvh,
-    int start, int end, int split, int nsplit, const int32_t* __restrict__ prow = nullptr) {
+    int start, int end, int split, int nsplit, const int32_t* __restrict__ prow = nullptr,
+    float* part = nullptr) {
   constexpr int QC = G * PR;      // query columns in use
   constexpr int KCH = D / 32;     // K . Q^T MFMA k-steps
   constexpr int DT = D / 16;      // output dim tiles of the P.V MFMA
@@ -502,6 +537,14 @@ __device__ __forceinline__ void decode_wave_mfma2(
     ohead = l16 % G;
     if (orow < 0) return;
   }
+  if constexpr (GROUP) {  // (the wave's own tiles: it has read them)
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+      *reinterpret_cast<float4*>(part + l16 * D + 16 * t + 4 * grp) =
+          make_float4(o[t][0], o[t][1], o[t][2], o[t][3]);
+    if (grp == 0) *reinterpret_cast<float2*>(part + G * D + 2 * l16) = make_float2(m, lsum);
+    return;
+  }
   const int64_t hidx = (int64_t)orow * num_q_heads + (int64_t)kvh * G + ohead;
   if (nsplit == 1) {
     const float inv = 1.f / lsum;
@@ -574,6 +617,81 @@ __attribute__((amdgpu_waves_per_eu((D == 128 && G * PR > 8) ? 2 : 3)))
   } else {
     run(std::integral_constant<bool, KV == 1>{});
   }
+}
+
+// Short contexts of unshared blocks (DecodePlanHost::groups): one workgroup of WAVES waves per
+// (row, KV head), a piece of the context per wave, merged through LDS in piece
+// order, so no partial result leaves the CU and no merge launch follows.  What
+// bounds such calls is latency: the launches, and the chain of a piece's steps.
+template <int D, int G, int WAVES>
+__device__ inline void group_merge(const float* parts, int stride, int n, int row, int kvh,
+                                   int num_q_heads, const AttnOut& out) {
+  for (int i = threadIdx.x; i < G * D; i += 64 * WAVES) {
+    const int g = i / D, d = i - g * D;
+    float mx = -INFINITY;
+    for (int s = 0; s < n; ++s) mx = fmaxf(mx, parts[s * stride + G * D + 2 * g]);
+    float l = 0.f, v = 0.f;
+    for (int s = 0; s < n; ++s) {
+      const float* p = parts + s * stride;
+      const float w = __expf(p[G * D + 2 * g] - mx);
+      l += w * p[G * D + 2 * g + 1];
+      v += w * p[i];
+    }
+    v *= 1.f / l;
+    if (out.frag)
+      store_frag(out.frag, out.mtiles, row, (kvh * G + g) * D + d, v);
+    else
+      out.rows[((int64_t)row * num_q_heads + kvh * G + g) * D + d] = v;
+  }
+}
+
+template <int D, int G, bool BIG_BLOCKS, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
+    paged_decode_group_kernel(const uint16_t* __restrict__ kv_layer, uint32_t blk_stride,
+                              uint32_t v_off, uint32_t slot_stride, uint32_t head_stride,
+                              int bs_log2, int num_kv_heads, int num_q_heads,
+                              const DecodeWork* __restrict__ work, const float* __restrict__ q,
+                              const uint32_t* __restrict__ bt_ids, float scale, AttnOut out) {
+  // per wave: V tile, query tile, K tile; then its partial result
+  constexpr int VT = 16 * (D + 8), QT = 2 * G * (D + 8), KT = 16 * D;
+  constexpr int kTile = VT + QT + KT;
+  static_assert(kTile / 2 >= group_part_floats<D, G>() && kTile % 8 == 0, "the part fits");
+  __shared__ __attribute__((aligned(16))) uint16_t lds[WAVES][kTile];
+  const int wv = threadIdx.x >> 6;
+  const DecodeWork wk = work[blockIdx.x * WAVES + wv];
+  const int row = wk.item / num_kv_heads, kvh = wk.item - row * num_kv_heads;
+  uint16_t* mine = lds[wv];
+  if (__builtin_amdgcn_readfirstlane(wk.end) > 0)
+    decode_wave_mfma2<D, G, true, BIG_BLOCKS, 1, true>(
+        kv_layer, blk_stride, v_off, slot_stride, head_stride, bs_log2, num_q_heads, q,
+        bt_ids + wk.tbl_off, wk.blk0, 1, scale, out, nullptr, nullptr, mine, mine + VT,
+        mine + VT + QT, row, kvh, wk.start, wk.end, 0, 1, nullptr,
+        reinterpret_cast<float*>(mine));
+  __syncthreads();
+  group_merge<D, G, WAVES>(reinterpret_cast<const float*>(lds), kTile / 2, wk.nsplit, row, kvh,
+                           num_q_heads, out);
+}
+
+template <typename T, int D, int G, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
+    paged_decode_group_valu_kernel(const T* __restrict__ kv_layer, int64_t blk_stride,
+                                   int64_t v_off, int64_t slot_stride, int64_t head_stride,
+                                   int bs_log2, int num_kv_heads, int num_q_heads,
+                                   const DecodeWork* __restrict__ work,
+                                   const float* __restrict__ q,
+                                   const uint32_t* __restrict__ bt_ids, float scale, AttnOut out) {
+  constexpr int kPart = (group_part_floats<D, G>() + 3) & ~3;
+  __shared__ __attribute__((aligned(16))) float parts[WAVES][kPart];
+  const int wv = threadIdx.x >> 6;
+  const DecodeWork wk = work[blockIdx.x * WAVES + wv];
+  const int row = wk.item / num_kv_heads, kvh = wk.item - row * num_kv_heads;
+  if (__builtin_amdgcn_readfirstlane(wk.end) > 0)
+    decode_wave_valu<T, D, G, true>(kv_layer, blk_stride, v_off, slot_stride, head_stride, bs_log2,
+                                    num_q_heads, q, bt_ids + wk.tbl_off, 1, scale, nullptr,
+                                    nullptr, nullptr, row, kvh, wk.start, wk.end, 0, 1,
+                                    parts[wv]);
+  __syncthreads();
+  group_merge<D, G, WAVES>(&parts[0][0], kPart, wk.nsplit, row, kvh, num_q_heads, out);
 }
 
 // Merges the per-split states of rows whose context spans several splits.
@@ -855,6 +973,66 @@ static hipError_t launch_valu(int G, dim3 grid, hipStream_t st, const T* kv, con
   return hipGetLastError();
 }
 
+template <int D, int WAVES>
+static hipError_t launch_group(int G, hipStream_t st, const uint16_t* kv, const ArenaStrides& a,
+                               int bsl, int hkv, int hq, const DecodePlanDev& plan,
+                               const float* q, const uint32_t* bi, float scale, bool big,
+                               const AttnOut& out) {
+  const dim3 grid((unsigned)plan.num_groups), block(64 * WAVES);
+#define ORION_GROUP_ARGS                                                                       \
+  grid, block, 0, st, kv, (uint32_t)a.blk, (uint32_t)a.v_off, (uint32_t)a.slot,                \
+      (uint32_t)a.head, bsl, hkv, hq, plan.groups, q, bi, scale, out
+#define ORION_GROUP_CASE(GG)                                                                   \
+  case GG:                                                                                     \
+    if (big)                                                                                   \
+      hipLaunchKernelGGL((paged_decode_group_kernel<D, GG, true, WAVES>), ORION_GROUP_ARGS);   \
+    else                                                                                       \
+      hipLaunchKernelGGL((paged_decode_group_kernel<D, GG, false, WAVES>), ORION_GROUP_ARGS);  \
+    break;
+  switch (G) {
+    ORION_GROUP_CASE(1)
+    ORION_GROUP_CASE(2)
+    ORION_GROUP_CASE(3)
+    ORION_GROUP_CASE(4)
+    ORION_GROUP_CASE(5)
+    ORION_GROUP_CASE(6)
+    ORION_GROUP_CASE(7)
+    ORION_GROUP_CASE(8)
+    default:
+      return hipErrorInvalidValue;
+  }
+#undef ORION_GROUP_CASE
+#undef ORION_GROUP_ARGS
+  return hipGetLastError();
+}
+
+template <int D>
+static hipError_t launch_group_valu(int G, hipStream_t st, const float* kv, const ArenaStrides& a,
+                                    int bsl, int hkv, int hq, const DecodePlanDev& plan,
+                                    const float* q, const uint32_t* bi, float scale,
+                                    const AttnOut& out) {
+#define ORION_GROUP_CASE(GG, WAVES)                                                            \
+  case GG:                                                                                     \
+    hipLaunchKernelGGL((paged_decode_group_valu_kernel<float, D, GG, WAVES>),                  \
+                       dim3((unsigned)plan.num_groups), dim3(64 * WAVES), 0, st, kv, a.blk,    \
+                       a.v_off, a.slot, a.head, bsl, hkv, hq, plan.groups, q, bi, scale, out); \
+    break;
+  switch (G) {  // (decode_group_waves: 16 waves where 128 registers hold one)
+    ORION_GROUP_CASE(1, kGroupWaves[1])
+    ORION_GROUP_CASE(2, kGroupWaves[1])
+    ORION_GROUP_CASE(3, kGroupWaves[1])
+    ORION_GROUP_CASE(4, kGroupWaves[1])
+    ORION_GROUP_CASE(5, kGroupWaves[0])
+    ORION_GROUP_CASE(6, kGroupWaves[0])
+    ORION_GROUP_CASE(7, kGroupWaves[0])
+    ORION_GROUP_CASE(8, kGroupWaves[0])
+    default:
+      return hipErrorInvalidValue;
+  }
+#undef ORION_GROUP_CASE
+  return hipGetLastError();
+}
+
 template <int D, int KV, bool BIG>
 static hipError_t launch_mfma2(int G, dim3 grid, hipStream_t st, const uint16_t* kv,
                                const ArenaStrides& a, int bsl, int hkv, int hq,
@@ -955,7 +1133,7 @@ hipError_t launch_paged_decode(hipStream_t st, const KvGeom& kv, const void* are
   float* ws_o = plan.ws;
   float* ws_ml = ws_o ? ws_o + rows * hq * ms * D : nullptr;
   if (phase == DecodePhase::kMerge) {
-    if (ms <= 1) return hipSuccess;
+    if (ms <= 1 || plan.num_groups) return hipSuccess;
     return launch_combine(st, D, rows, hq, plan, ms, ws_o, ws_ml, out);
   }
   int bs_log2 = 0;
@@ -964,6 +1142,23 @@ hipError_t launch_paged_decode(hipStream_t st, const KvGeom& kv, const void* are
   const float scale = 1.0f / sqrtf((float)D);
   const dim3 grid((unsigned)((plan.num_work + 3) / 4));
   hipError_t e;
+  if (plan.num_groups) {  // one launch, the plan's shape (build_decode_groups)
+    const bool wide = plan.group_waves == kGroupWaves[1];
+    if (G > 8 || (D != 64 && D != 128) || a.blk > (int64_t)UINT32_MAX ||
+        plan.group_waves != decode_group_waves(kv, hq))
+      return hipErrorInvalidValue;
+    if (kv.dtype_bf16) {
+      const uint16_t* base = static_cast<const uint16_t*>(arena) + layer * a.layer;
+      const bool big = kv.block_size >= 16;
+      return wide ? launch_group<64, kGroupWaves[1]>(G, st, base, a, bs_log2, (int)hkv, (int)hq,
+                                                     plan, q, bt_ids, scale, big, out)
+                  : launch_group<128, kGroupWaves[0]>(G, st, base, a, bs_log2, (int)hkv, (int)hq,
+                                                      plan, q, bt_ids, scale, big, out);
+    }
+    const float* base = static_cast<const float*>(arena) + layer * a.layer;
+    return launch_group_valu<64>(G, st, base, a, bs_log2, (int)hkv, (int)hq, plan, q, bt_ids,
+                                 scale, out);
+  }
   // bf16 arenas at head_dim 64/128 with up to 16 query heads per KV head (the
   // MFMA B operand's 16 columns) take the MFMA wave; f32 arenas take the VALU
   // wave up to 8; everything else the general wave.

@@ -383,6 +383,68 @@ int decode_pack_rows(const KvGeom& kv, int64_t hq) {
   return G >= 1 && G <= 8 ? (int)(16 / G) : 0;
 }
 
+int decode_group_waves(const KvGeom& kv, int64_t hq) {
+  if (kv.num_kv_heads <= 0) return 0;
+  const int64_t G = hq / kv.num_kv_heads;
+  if (G < 1 || G > 8) return 0;
+  if (kv.dtype_bf16) return kv.head_dim == 64 ? kGroupWaves[1] : kv.head_dim == 128 ? kGroupWaves[0] : 0;
+  return kv.head_dim == 64 ? kGroupWaves[G <= 4] : 0;
+}
+
+// Longest piece of a grouped row: two 16-token steps, or four where bf16 rows
+// are at most a pair per four CUs (the f32 wave holds two).  Against separate
+// items and merge, one row of up to 500 tokens took 5.3 us for 8.7 (bf16,
+// head_dim 64, 4 KV heads) and 6.3 for 10.9 (f32), 32 rows of them 7.4 for 8.5,
+// and 4 rows of up to 500 at head_dim 128, 8 KV heads, 8.7 for 9.5.  With four
+// steps a wave for more pairs, 32 rows of up to 1000 tokens took 10.1 us for 9.9
+// and a 22-layer step of them 1607 for 1567: there the pieces over all CUs are
+// worth the merge launch, as they are with more (row, KV head) pairs than CUs.
+constexpr int kGroupPiece = 32;
+
+void build_decode_groups(const uint32_t* positions, const int32_t* row_seq,
+                         const int64_t* bt_offsets, const uint32_t* bt_ids, int64_t rows,
+                         int64_t hkv, int64_t block_size, int64_t cus, int group_waves, bool bf16,
+                         const uint8_t* skip_rows, DecodePlanHost* plan) {
+  plan->groups.clear();
+  plan->group_waves = 0;
+  // ORION_DECODE_GROUP=0 keeps the separate items and merge (read per call, so a
+  // test can run one batch both ways)
+  const char* env = getenv("ORION_DECODE_GROUP");
+  if (env && env[0] == '0') return;
+  // (a plan without splits runs in one launch already; rows that share blocks
+  // keep the cached loads of separate items, packed or not)
+  if (!group_waves || !plan->stream_kv || plan->max_splits <= 1) return;
+  const int64_t unit = std::max<int64_t>(16, block_size);
+  int64_t planned = 0, longest = 0;
+  for (int64_t r = 0; r < rows; ++r) {
+    if (skip_rows && skip_rows[r]) continue;
+    ++planned;
+    longest = std::max<int64_t>(longest, (int64_t)positions[r] + 1);
+  }
+  const int64_t longest_piece = bf16 && planned * hkv * 4 <= cus ? 2 * kGroupPiece : kGroupPiece;
+  if (planned * hkv > cus || longest > longest_piece * group_waves || unit > longest_piece)
+    return;
+  plan->group_waves = group_waves;
+  plan->groups.reserve((size_t)(planned * hkv * group_waves));
+  for (int64_t r = 0; r < rows; ++r) {
+    if (skip_rows && skip_rows[r]) continue;
+    const int64_t L = (int64_t)positions[r] + 1;
+    const int64_t piece = ((L + group_waves - 1) / group_waves + unit - 1) / unit * unit;
+    const int32_t n = (int32_t)((L + piece - 1) / piece);
+    const int64_t table = bt_offsets[row_seq[r]];
+    for (int64_t h = 0; h < hkv; ++h)
+      for (int s = 0; s < group_waves; ++s) {
+        const int64_t start = s * piece, end = std::min(L, start + piece);
+        const int64_t at = table + start / block_size;
+        if (s < n)
+          plan->groups.push_back({(int32_t)(r * hkv + h), (int32_t)start, (int32_t)end, n,
+                                  (int32_t)at, (int32_t)bt_ids[at], 0, s});
+        else
+          plan->groups.push_back({(int32_t)(r * hkv + h), 0, 0, n, 0, 0, 0, s});
+      }
+  }
+}
+
 size_t decode_workspace_bytes(int64_t rows, int64_t hq, int64_t D, int64_t max_splits) {
   if (max_splits <= 1) return 0;
   return (size_t)(rows * hq * max_splits) * (size_t)(D + 2) * sizeof(float);

@@ -81,6 +81,11 @@ struct DecodePlanHost {
   int num_packed = 0;
   int pack_r = 0;
   std::vector<int32_t> pack_rows;
+  // Short contexts: group_waves items per (row, KV head), run and merged by one
+  // workgroup instead of `work` and the merge launch (build_decode_groups; end
+  // 0: no piece, nsplit: the row's pieces).
+  int group_waves = 0;
+  std::vector<DecodeWork> groups;
 };
 struct DecodePlanDev {
   const DecodeWork* work = nullptr;
@@ -99,6 +104,10 @@ struct DecodePlanDev {
   int num_packed = 0;
   const int32_t* pack_rows = nullptr;
   int pack_r = 0;
+  // DecodePlanHost::groups on the device; num_groups workgroups of group_waves
+  const DecodeWork* groups = nullptr;
+  int num_groups = 0;
+  int group_waves = 0;
 };
 // pack_r: rows per packed prefix item; 0 packs nothing.  The decode kernels
 // take packed items only on bf16 arenas at head_dim 64/128 with
@@ -107,6 +116,17 @@ void build_decode_plan(const uint32_t* positions, const int32_t* row_seq,
                        const int64_t* bt_offsets, const uint32_t* bt_ids, int64_t rows,
                        int64_t hkv, int64_t block_size, int64_t wave_slots,
                        const uint8_t* skip_rows, DecodePlanHost* plan, int pack_r = 0);
+// Waves per workgroup of a grouped plan: 16 where a wave fits 128 registers
+// (head_dim 64; f32 arenas up to 4 query heads per KV head), else 8; 0 where the
+// group kernels do not apply (they lost on f32 arenas at head_dim 128).
+constexpr int kGroupWaves[2] = {8, 16};
+int decode_group_waves(const KvGeom& kv, int64_t hq);
+// Fills plan->groups when the planned rows are few and short enough
+// (group_waves of 0 leaves the plan as it is).
+void build_decode_groups(const uint32_t* positions, const int32_t* row_seq,
+                         const int64_t* bt_offsets, const uint32_t* bt_ids, int64_t rows,
+                         int64_t hkv, int64_t block_size, int64_t cus, int group_waves, bool bf16,
+                         const uint8_t* skip_rows, DecodePlanHost* plan);
 size_t decode_workspace_bytes(int64_t rows, int64_t hq, int64_t D, int64_t max_splits);
 // Rows per packed prefix item for this arena and grouping (0: no packing).
 int decode_pack_rows(const KvGeom& kv, int64_t hq);

@@ -213,9 +213,9 @@ struct orion_hip_decode_plan {
   orion_hip_device* dev = nullptr;
   int64_t rows = 0, hq = 0, hkv = 0, head_dim = 0, block_size = 0;
   // host: the plan as built for a bf16 arena (shared prefixes packed where
-  // the MFMA wave takes them); plain: the same rows without packing, built
-  // only when host packs something (an f32 arena takes it).  Each device
-  // buffer holds the work items, the pieces per row, then the pack rows.
+  // the MFMA wave takes them); plain: the same rows as an f32 arena takes
+  // them, built when that differs.  Each device buffer holds the work items,
+  // the pieces per row, the pack rows, then the groups.
   DecodePlanHost host, plain;
   DevBuf work, work_plain, ws;
   ~orion_hip_decode_plan() {
@@ -237,10 +237,20 @@ struct orion_hip_decode_plan {
     d.pack_rows = reinterpret_cast<const int32_t*>(base + h.work.size() * sizeof(DecodeWork) +
                                                    h.row_nsplit.size() * sizeof(int32_t));
     d.pack_r = h.pack_r;
+    d.groups = reinterpret_cast<const DecodeWork*>(base + groups_at(h));
+    d.group_waves = h.group_waves;
+    d.num_groups = h.group_waves ? (int)(h.groups.size() / h.group_waves) : 0;
     return d;
   }
+  // Byte offset of the groups, after the pack rows.
+  static size_t groups_at(const DecodePlanHost& h) {
+    return (h.work.size() * sizeof(DecodeWork) + h.row_nsplit.size() * 4 + h.pack_rows.size() * 4 +
+            15) & ~(size_t)15;
+  }
+  // f32 arenas take no packs, and groups of another size
+  bool has_plain() const { return host.num_packed || host.group_waves; }
   DecodePlanDev view(bool bf16) const {
-    DecodePlanDev d = (!bf16 && host.num_packed) ? view_of(plain, work_plain) : view_of(host, work);
+    DecodePlanDev d = (!bf16 && has_plain()) ? view_of(plain, work_plain) : view_of(host, work);
     d.ws = ws.as<float>();
     d.ws_bytes = ws.bytes;
     return d;
@@ -1578,6 +1588,10 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
     build_decode_plan(b->positions, hb.row_seq.data(), b->block_table_offsets,
                       b->block_table_ids, n, d.num_kv_heads, d.block_size, m->dev->wave_slots,
                       npf ? skip.data() : nullptr, &plan, decode_pack_rows(m->kv, Hq));
+    build_decode_groups(b->positions, hb.row_seq.data(), b->block_table_offsets,
+                        b->block_table_ids, n, d.num_kv_heads, d.block_size,
+                        m->dev->wave_slots / 8, decode_group_waves(m->kv, Hq), m->kv.dtype_bf16,
+                        npf ? skip.data() : nullptr, &plan);
     // One workspace for the decode splits and the prefill key parts (their
     // launches are ordered on the stream: the decode merge has read the
     // splits before the prefill kernel writes its parts).
@@ -1595,7 +1609,8 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
     const size_t o_pfsplit = o_pforder + pf_order.size() * sizeof(PrefillTile);
     const size_t o_pfparts = o_pfsplit + (pf_split ? pfp.split_rows.size() * 4 : 0);
     const size_t o_packrows = o_pfparts + (pf_split ? pfp.row_parts.size() * 4 : 0);
-    const size_t ptotal = std::max<size_t>(o_packrows + plan.pack_rows.size() * 4, 8);
+    const size_t o_groups = (o_packrows + plan.pack_rows.size() * 4 + 15) & ~(size_t)15;
+    const size_t ptotal = std::max<size_t>(o_groups + plan.groups.size() * sizeof(DecodeWork), 8);
     HIP_TRY(st, m->h_plan.reserve(ptotal));
     HIP_TRY(st, m->b_plan.reserve(ptotal));
     char* hp = static_cast<char*>(m->h_plan.ptr);
@@ -1612,6 +1627,7 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
       std::memcpy(hp + o_pfparts, pfp.row_parts.data(), pfp.row_parts.size() * 4);
     }
     std::memcpy(hp + o_packrows, plan.pack_rows.data(), plan.pack_rows.size() * 4);
+    std::memcpy(hp + o_groups, plan.groups.data(), plan.groups.size() * sizeof(DecodeWork));
     char* pp = m->b_plan.as<char>();
     HIP_TRY(st, upload(stream, pp, hp, ptotal));
     dplan.work = reinterpret_cast<const DecodeWork*>(pp + o_work);
@@ -1626,6 +1642,9 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
     dplan.num_packed = plan.num_packed;
     dplan.pack_rows = reinterpret_cast<const int32_t*>(pp + o_packrows);
     dplan.pack_r = plan.pack_r;
+    dplan.groups = reinterpret_cast<const DecodeWork*>(pp + o_groups);
+    dplan.group_waves = plan.group_waves;
+    dplan.num_groups = plan.group_waves ? (int)(plan.groups.size() / plan.group_waves) : 0;
     if (npf) {
       dplan.rows = reinterpret_cast<const int32_t*>(pp + o_drows);
       dplan.num_rows = (int)plan.rows.size();
@@ -1911,27 +1930,39 @@ ORION_EXPORT int orion_hip_decode_plan_create(orion_hip_device* dev, const uint3
   const int pack_r = decode_pack_rows(bf16_geom, num_q_heads);
   build_decode_plan(positions, row_seq, block_table_offsets, block_table_ids, num_rows,
                     num_kv_heads, block_size, dev->wave_slots, nullptr, &p->host, pack_r);
-  if (p->host.num_packed)
+  const KvGeom f32_geom{1, 1, block_size, num_kv_heads, head_dim, false};
+  auto group = [&](const KvGeom& geom, DecodePlanHost* h) {
+    build_decode_groups(positions, row_seq, block_table_offsets, block_table_ids, num_rows,
+                        num_kv_heads, block_size, dev->wave_slots / 8,
+                        decode_group_waves(geom, num_q_heads), geom.dtype_bf16, nullptr, h);
+  };
+  group(bf16_geom, &p->host);
+  if (p->has_plain()) {
     build_decode_plan(positions, row_seq, block_table_offsets, block_table_ids, num_rows,
                       num_kv_heads, block_size, dev->wave_slots, nullptr, &p->plain, 0);
+    group(f32_geom, &p->plain);
+  }
   // work items, then the pieces per row, then the pack rows, in one buffer
   auto upload = [&](const DecodePlanHost& h, DevBuf& buf) -> hipError_t {
     const size_t wbytes = h.work.size() * sizeof(DecodeWork);
     const size_t nbytes = h.row_nsplit.size() * sizeof(int32_t);
     const size_t pbytes = h.pack_rows.size() * sizeof(int32_t);
-    hipError_t e = buf.reserve(wbytes + nbytes + pbytes);
+    const size_t o_groups = orion_hip_decode_plan::groups_at(h);
+    const size_t total = o_groups + h.groups.size() * sizeof(DecodeWork);
+    hipError_t e = buf.reserve(total);
     if (e != hipSuccess) return e;
-    std::vector<char> staged(wbytes + nbytes + pbytes);
+    std::vector<char> staged(total);
     std::memcpy(staged.data(), h.work.data(), wbytes);
     std::memcpy(staged.data() + wbytes, h.row_nsplit.data(), nbytes);
     std::memcpy(staged.data() + wbytes + nbytes, h.pack_rows.data(), pbytes);
+    std::memcpy(staged.data() + o_groups, h.groups.data(), h.groups.size() * sizeof(DecodeWork));
     if (staged.empty()) return hipSuccess;
     e = hipMemcpyAsync(buf.ptr, staged.data(), staged.size(), hipMemcpyHostToDevice, dev->stream);
     if (e != hipSuccess) return e;
     return hipStreamSynchronize(dev->stream);  // staged is freed on return
   };
   HIP_TRY(st, upload(p->host, p->work));
-  if (p->host.num_packed) HIP_TRY(st, upload(p->plain, p->work_plain));
+  if (p->has_plain()) HIP_TRY(st, upload(p->plain, p->work_plain));
   HIP_TRY(st, p->ws.reserve(decode_workspace_bytes(
                   num_rows, num_q_heads, head_dim,
                   std::max(p->host.max_splits, p->plain.max_splits))));
