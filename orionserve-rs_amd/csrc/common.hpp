@@ -46,6 +46,7 @@ constexpr int kDppXor1 = 0xB1;
 constexpr int kDppXor2 = 0x4E;
 constexpr int kDppHalfMirror = 0x141;
 constexpr int kDppMirror = 0x140;
+constexpr int kDppRor8 = 0x128;  // lane i takes lane (i + 8) % 16's
 
 // Sum over groups of N consecutive lanes (N in 1..64, power of two); every
 // lane of a group ends with the group total.
@@ -156,5 +157,12 @@ __device__ inline void lds_load16(const void* src, uint32_t lds_wave_base) {
 
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima).
 __device__ inline void wait_vmem_all() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+// s_waitcnt vmcnt(N): all but the wave's N newest vector memory operations are
+// done (they retire in order); the count is split over bits 3:0 and 15:14.
+template <int N>
+__device__ inline void wait_vmem() {
+  static_assert(N >= 0 && N < 64, "a 6-bit count");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
 
 }  // namespace orion

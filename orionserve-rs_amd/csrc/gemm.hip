@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
+#include <type_traits>
 #include <utility>
 
 namespace orion {
@@ -192,7 +193,7 @@ __global__ void __launch_bounds__(64 * KW)
 // fragments by the 4 column tiles.  LDS rows are XOR-swizzled in 16-byte
 // chunks (conflict-free 16-byte fragment reads; the DMA writes stay linear).
 namespace {
-constexpr int kTM = 128, kTN = 128, kTK = 32;
+constexpr int kTN = 128, kTK = 32;
 // A tile row r: 8 chunks of 4 floats; chunk c stored at c ^ swz_a(r).
 __device__ inline int swz_a(int r) {
   return ((r >> 2) & 1) | (((r >> 1) & 1) << 1) | (((r >> 3) & 1) << 2);
@@ -210,23 +211,100 @@ struct PackedGeom {
   int pair_dim = 0, pair_cols = 0;  // packed_column
 };
 
+// The QKV tile of a wave with RoPE and the cache write (a prefill-shaped
+// forward's): columns 2j and 2j + 1 of 16 hold 16 columns of a head's first half
+// and the 16 they rotate with, 8 and 8 of each (packed_column), so one exchange
+// within 16 lanes leaves a lane both of a pair and every store 16 consecutive
+// elements.  The same f32 expressions as rope_cache_kernel.  As a kernel of its
+// own RoPE re-read the f32 QKV matrix, 60 us at 17631 rows of 2560 columns, and
+// storing that matrix from this column order took 22 us more; the GEMM with both
+// takes 353 us.
+template <int MTW, int NTW>
+__device__ inline void rope_tiles(const RopeOut& r, const f32x4 (&acc)[MTW][NTW],
+                                  const RowSlot* slots, int row0, int col0, int M, int N, int D,
+                                  const float* __restrict__ bias) {
+#pragma clang fp contract(off)
+  const int l16 = threadIdx.x & 15, grp = (threadIdx.x & 63) >> 4;
+  const int half = D >> 1;
+  const float* __restrict__ cos_t = r.cos;
+  const float* __restrict__ sin_t = r.sin;
+#pragma unroll
+  for (int nt = 0; nt < NTW; nt += 2) {
+    const int c = col0 + 16 * nt;  // 32 columns of one head (D is a multiple of 32)
+    if (c >= N) continue;
+    const int unit = c / D, at = c - unit * D;
+    if (unit >= r.hq + r.hkv) {  // V: as it is
+      const int64_t to = r.v_off + (int64_t)(unit - r.hq - r.hkv) * r.head + at + l16;
+      const float b0 = bias ? bias[c + l16] : 0.f, b1 = bias ? bias[c + 16 + l16] : 0.f;
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int rl = mt * 16 + 4 * grp + i;
+          float v0 = acc[mt][nt][i], v1 = acc[mt][nt + 1][i];
+          if (bias) v0 = v0 + b0, v1 = v1 + b1;
+          if (row0 + rl < M) {
+            store_kv1(r.kv, r.kv_bf16, slots[rl].kv + to, v0);
+            store_kv1(r.kv, r.kv_bf16, slots[rl].kv + to + 16, v1);
+          }
+        }
+      continue;
+    }
+    const int j = (at >> 1) + l16;  // of the first half
+    const bool q = unit < r.hq;
+    const int64_t k_to = (int64_t)(unit - r.hq) * r.head + j;
+    const float b0 = bias ? bias[unit * D + j] : 0.f, b1 = bias ? bias[unit * D + half + j] : 0.f;
+#pragma unroll
+    for (int mt = 0; mt < MTW; ++mt) {
+      float cs[4], sn[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t a = (int64_t)slots[mt * 16 + 4 * grp + i].pos * half + j;
+        cs[i] = cos_t[a];
+        sn[i] = sin_t[a];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int rl = mt * 16 + 4 * grp + i;
+        const float even = acc[mt][nt][i], odd = acc[mt][nt + 1][i];
+        const float got = dpp<kDppRor8>(l16 < 8 ? odd : even);
+        float x0 = l16 < 8 ? even : got, x1 = l16 < 8 ? got : odd;
+        if (bias) x0 = x0 + b0, x1 = x1 + b1;
+        const float y0 = x0 * cs[i] - x1 * sn[i], y1 = x0 * sn[i] + x1 * cs[i];
+        if (row0 + rl >= M) continue;
+        if (q) {
+          float* to = r.q_out + ((int64_t)(row0 + rl) * r.hq + unit) * D + j;
+          to[0] = y0;
+          to[half] = y1;
+        } else {
+          store_kv1(r.kv, r.kv_bf16, slots[rl].kv + k_to, y0);
+          store_kv1(r.kv, r.kv_bf16, slots[rl].kv + k_to + half, y1);
+        }
+      }
+    }
+  }
+}
+
 // HILO: x carried as a truncated hi + lo bf16 pair (two MFMAs, ~16 bits of
 // x per product); otherwise rounded to bf16 (nearest even, one MFMA).
 // XS (with HILO): x is already in that split layout (GemmFuse::x_hilo), so a
 // fragment's two 16-byte LDS chunks are its hi and lo bf16x8 as they are.
 // NTW: 16-column tiles per wave (4: 128-column workgroup tiles; 8: 256).
 // out_hilo: the SwiGLU epilogue writes its output in the split layout.
-template <bool HILO, int NTW, bool XS = false>
+// MTW: 16-row tiles per wave (TM = 32 MTW workgroup rows).  ST: k-step tiles in
+// LDS (see the loop).  ROPE: the QKV GEMM, whose epilogue is rope's.
+template <bool HILO, int NTW, bool XS = false, int MTW = 4, int ST = 2, bool ROPE = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW == 8 ? 2 : 1)))
     gemm_tiled_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
                       const float* __restrict__ bias, int M, int N, int K, int ep,
                       float* __restrict__ out, PackedGeom pk, int gm, int kspan,
-                      float* __restrict__ partial, bool out_hilo) {
+                      float* __restrict__ partial, bool out_hilo, RopeOut rope) {
   static_assert(HILO || !XS, "a pre-split x needs the hi/lo MFMAs");
+  constexpr int TM = 32 * MTW;   // workgroup rows
   constexpr int TN = 32 * NTW;   // workgroup columns
   constexpr int BJ = NTW / 2;    // B copies (1 KiB each) per wave per k-step
-  __shared__ __attribute__((aligned(1024))) float As[2][kTM * kTK];
-  __shared__ __attribute__((aligned(1024))) uint16_t Bs[2][TN * kTK];
+  __shared__ __attribute__((aligned(1024))) float As[ST][TM * kTK];
+  __shared__ __attribute__((aligned(1024))) uint16_t Bs[ST][TN * kTK];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -240,7 +318,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
   // tiles in flight on one XCD share A and B slabs in its L2.
   int mt_i = blockIdx.y, nt_i = blockIdx.x;
   if (gm > 0) {
-    const int gx = (N + TN - 1) / TN, gy = (M + kTM - 1) / kTM, total = gx * gy;
+    const int gx = (N + TN - 1) / TN, gy = (M + TM - 1) / TM, total = gx * gy;
     const int b = blockIdx.x;
     const int per = (total + 7) / 8;
     const int t = (b & 7) * per + (b >> 3);
@@ -250,15 +328,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
     mt_i = g * gm + within % gm_eff;
     nt_i = within / gm_eff;
   }
-  const int m0 = mt_i * kTM, n0 = nt_i * TN;
+  const int m0 = mt_i * TM, n0 = nt_i * TN;
 
-  // ---- DMA addressing: A = 4 wave instructions (8 rows x 128 B each),
-  // B = 2 wave instructions (16 rows x 64 B each). ----
-  const float* a_src[4];
+  // ---- DMA addressing: A = MTW wave instructions (8 rows x 128 B each),
+  // B = BJ wave instructions (16 rows x 64 B each). ----
+  const float* a_src[MTW];
   const uint16_t* b_src[BJ];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int r = (wave * 4 + j) * 8 + (lane >> 3);
+  for (int j = 0; j < MTW; ++j) {
+    const int r = (wave * MTW + j) * 8 + (lane >> 3);
     const int c = (lane & 7) ^ swz_a(r);
     a_src[j] = x + (int64_t)min(m0 + r, M - 1) * K + c * 4;
   }
@@ -283,21 +361,28 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
   auto load_tile = [&](int ks, int buf) {
     const int k0 = ks * kTK;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      lds_load16(a_src[j] + k0, as_base + (uint32_t)(buf * kTM * kTK * 4 + (wave * 4 + j) * 1024));
+    for (int j = 0; j < MTW; ++j)
+      lds_load16(a_src[j] + k0, as_base + (uint32_t)(buf * TM * kTK * 4 + (wave * MTW + j) * 1024));
 #pragma unroll
     for (int j = 0; j < BJ; ++j)
       lds_load16(b_src[j] + (int64_t)ks * b_step,
                  bs_base + (uint32_t)(buf * TN * kTK * 2 + (wave * BJ + j) * 1024));
   };
 
+  // where each row's K and V go, and its position: read while the first tiles load
+  __shared__ RowSlot slots[ROPE ? TM : 1];
+  auto find_slots = [&] {
+    if constexpr (ROPE)
+      if (tid < TM) slots[tid] = row_slot(rope, min(m0 + tid, M - 1));
+  };
+
   // ---- fragment read addresses (bytes, buffer 0) ----
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-  uint32_t a_rd0[4], a_rd1[4], b_rd[NTW];
+  uint32_t a_rd0[MTW], a_rd1[MTW], b_rd[NTW];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int r = wm * 64 + mt * 16 + l16;
+  for (int mt = 0; mt < MTW; ++mt) {
+    const int r = wm * 16 * MTW + mt * 16 + l16;
     a_rd0[mt] = as_base + (uint32_t)(r * kTK + (((2 * grp) ^ swz_a(r)) * 4)) * 4;
     a_rd1[mt] = as_base + (uint32_t)(r * kTK + (((2 * grp + 1) ^ swz_a(r)) * 4)) * 4;
   }
@@ -308,29 +393,49 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
                       : bs_base + (uint32_t)(n * kTK + ((grp ^ swz_b(n)) * 8)) * 2;
   }
 
-  f32x4 acc[4][NTW];
+  f32x4 acc[MTW][NTW];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
     for (int nt = 0; nt < NTW; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // K split z = blockIdx.z covers k-steps [z * kspan, min(ksteps, (z + 1) * kspan))
   const int ks_begin = blockIdx.z * kspan;
   const int ksteps = min(K / kTK, ks_begin + kspan);
-  load_tile(ks_begin, 0);
-  wait_vmem_all();
-  __syncthreads();
+  // ST - 1 k-steps in flight.  A k-step's copies are this wave's MTW + BJ
+  // newest but (ST - 2) k-steps'; the barrier makes every wave's visible, and
+  // says that all have read the tile the next copies overwrite.
+  if constexpr (ST > 2) {
+#pragma unroll
+    for (int s = 0; s < ST - 1; ++s)
+      if (ks_begin + s < ksteps) load_tile(ks_begin + s, s);
+    find_slots();
+  } else {
+    load_tile(ks_begin, 0);
+    find_slots();
+    wait_vmem_all();
+    __syncthreads();
+  }
+  int buf = 0;
   for (int ks = ks_begin; ks < ksteps; ++ks) {
-    const int buf = (ks - ks_begin) & 1;
-    if (ks + 1 < ksteps) load_tile(ks + 1, buf ^ 1);
-    const uint32_t aoff = (uint32_t)(buf * kTM * kTK * 4);
+    if constexpr (ST > 2) {
+      if (ks + ST - 2 < ksteps)
+        wait_vmem<(ST - 2) * (MTW + BJ)>();
+      else
+        wait_vmem_all();
+      __syncthreads();
+      if (ks + ST - 1 < ksteps) load_tile(ks + ST - 1, buf ? buf - 1 : ST - 1);
+    } else if (ks + 1 < ksteps) {
+      load_tile(ks + 1, buf ^ 1);
+    }
+    const uint32_t aoff = (uint32_t)(buf * TM * kTK * 4);
     const uint32_t boff = (uint32_t)(buf * TN * kTK * 2);
     bf16x8 bw[NTW];
 #pragma unroll
     for (int nt = 0; nt < NTW; ++nt)
       bw[nt] = __builtin_bit_cast(bf16x8, *(const lds_u32x4*)(uintptr_t)(b_rd[nt] + boff));
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
+    for (int mt = 0; mt < MTW; ++mt) {
       const u32x4 lo4 = *(const lds_u32x4*)(uintptr_t)(a_rd0[mt] + aoff);
       const u32x4 hi4 = *(const lds_u32x4*)(uintptr_t)(a_rd1[mt] + aoff);
       const float a[8] = {__uint_as_float(lo4.x), __uint_as_float(lo4.y),
@@ -359,11 +464,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
               __builtin_amdgcn_mfma_f32_16x16x32_bf16(alo, bw[nt], acc[mt][nt], 0, 0, 0);
       }
     }
-    wait_vmem_all();
-    __syncthreads();
+    if constexpr (ST > 2) {
+      buf = buf + 1 < ST ? buf + 1 : 0;
+    } else {
+      wait_vmem_all();
+      __syncthreads();
+      buf ^= 1;
+    }
   }
 
-  // ---- epilogue: acc[mt][nt][i] = C[m0 + wm*64 + mt*16 + 4*grp + i][n0 + wn*64 + nt*16 + l16] ----
+  // ---- epilogue: acc[mt][nt][i] = C[m0 + wm*16*MTW + mt*16 + 4*grp + i][n0 + wn*16*NTW + nt*16 + l16] ----
+  if constexpr (ROPE) {
+    rope_tiles<MTW, NTW>(rope, acc, slots + wm * 16 * MTW, m0 + wm * 16 * MTW, n0 + wn * 16 * NTW, M,
+                         N, pk.pair_dim, bias);
+    return;
+  }
   if (partial) {  // one K split: raw sums, reduced by gemm_tiled_reduce_kernel
     float* pz = partial + (int64_t)blockIdx.z * M * N;
 #pragma unroll
@@ -371,10 +486,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
       const int col = n0 + wn * 16 * NTW + nt * 16 + l16;
       const int oc = packed_column(col, pk.pair_dim, pk.pair_cols);
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int row = m0 + wm * 64 + mt * 16 + 4 * grp + i;
+          const int row = m0 + wm * 16 * MTW + mt * 16 + 4 * grp + i;
           if (row < M && col < N) pz[(int64_t)row * N + oc] = acc[mt][nt][i];
         }
     }
@@ -387,10 +502,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
       const int oc = packed_column(col, pk.pair_dim, pk.pair_cols);
       const float b = bias && col < N ? bias[oc] : 0.f;
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int row = m0 + wm * 64 + mt * 16 + 4 * grp + i;
+          const int row = m0 + wm * 16 * MTW + mt * 16 + 4 * grp + i;
           if (row < M && col < N) out[(int64_t)row * N + oc] = bias ? acc[mt][nt][i] + b : acc[mt][nt][i];
         }
     }
@@ -405,14 +520,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
     // launch.  (Loading the whole tile at once, or before the k-loop, takes
     // the kernel past the registers of three workgroups per CU.)
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
+    for (int mt = 0; mt < MTW; ++mt) {
       float res[NTW][4];
 #pragma unroll
       for (int nt = 0; nt < NTW; ++nt) {
         const int col = n0 + wn * 16 * NTW + nt * 16 + l16;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int row = m0 + wm * 64 + mt * 16 + 4 * grp + i;
+          const int row = m0 + wm * 16 * MTW + mt * 16 + 4 * grp + i;
           res[nt][i] = (row < M && col < N) ? out[(int64_t)row * N + col] : 0.f;
         }
       }
@@ -421,7 +536,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
         const int col = n0 + wn * 16 * NTW + nt * 16 + l16;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int row = m0 + wm * 64 + mt * 16 + 4 * grp + i;
+          const int row = m0 + wm * 16 * MTW + mt * 16 + 4 * grp + i;
           if (row < M && col < N) out[(int64_t)row * N + col] = res[nt][i] + acc[mt][nt][i];
         }
       }
@@ -429,13 +544,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
     return;
   }
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
+  for (int mt = 0; mt < MTW; ++mt) {
 #pragma unroll
     for (int nt = 0; nt < NTW; ++nt) {
       const int col = n0 + wn * 16 * NTW + nt * 16 + l16;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int row = m0 + wm * 64 + mt * 16 + 4 * grp + i;
+        const int row = m0 + wm * 16 * MTW + mt * 16 + 4 * grp + i;
         const float v = acc[mt][nt][i];
         // kSwiGLU: tile columns [0, 8) are gate rows of W, [8, 16) the matching
         // up rows.
@@ -794,6 +909,7 @@ void launch_gemv(const GemvShape& g, hipStream_t st, const float* x, const uint1
 namespace {
 constexpr int64_t kTiledFill = 256;
 constexpr int64_t kTiledSlots = 768;
+constexpr int64_t kTM = 128;  // rows of a tile, for the counts below
 int tiled_ksplits(int64_t M, int64_t N, int64_t K, bool preferred = true) {
   const int64_t tiles = ((N + kTN - 1) / kTN) * ((M + kTM - 1) / kTM);
   const int64_t ksteps = K / kTK;
@@ -810,13 +926,93 @@ int tiled_ksplits(int64_t M, int64_t N, int64_t K, bool preferred = true) {
   }
   return s;
 }
+
+// Workgroup tiles of the LDS-tiled GEMM: 32 mtw rows x 32 ntw columns, st
+// k-steps in LDS, `per_cu` workgroups resident (LDS and registers).  Up to
+// kShapeRows rows the grid is a few workgroups per CU, and what a GEMM takes is
+// its k-steps in a row times what one costs: `alone` us where the CU holds one
+// workgroup (latency; with two k-steps in LDS one copy is in flight, and it
+// is waited for) or `each` us per resident one where they fill the matrix cores.
+// Measured at 65 to 743 rows of N 4096, 6144 and 28672, K 4096 and 14336; the
+// estimate from these was within 15 % of each time.  160 rows, us before (128
+// rows and two k-steps in LDS; 256 columns at N 28672) and now: QKV 6144 x 4096
+// 38 -> 31, O 4096 x 4096 36 -> 25, gate/up 28672 x 4096 133 -> 85, down 4096 x
+// 14336 62 -> 48; 743 rows: QKV 105 -> 72, O 67 -> 56, gate/up 273 -> 240, down
+// 155 -> 140.
+struct TiledShape {
+  int ntw, mtw, st, per_cu;
+  float alone, each;
+};
+constexpr TiledShape kTiledShapes[] = {
+    {4, 4, 2, 3, 0.82f, 0.35f}, {4, 4, 3, 2, 0.54f, 0.40f}, {4, 3, 2, 4, 0.77f, 0.275f},
+    {4, 3, 3, 2, 0.47f, 0.335f}, {4, 2, 4, 2, 0.33f, 0.25f}, {4, 5, 3, 1, 0.66f, 0.66f},
+};
+constexpr TiledShape kTiledWide = {8, 4, 2, 2, 0.f, 0.f};
+constexpr int64_t kShapeRows = 1024;
+constexpr int kCus = 256;
+
+// Microseconds of a GEMM on shape t in `splits` K splits: rounds of per_cu
+// workgroups, each with a start and an end, and the sums' round trip and launch.
+float tiled_cost(const TiledShape& t, int64_t M, int64_t N, int64_t K, int splits) {
+  const int64_t wgs = ((M + 32 * t.mtw - 1) / (32 * t.mtw)) * ((N + 32 * t.ntw - 1) / (32 * t.ntw)) * splits;
+  const int64_t per = (wgs + kCus - 1) / kCus, full = per / t.per_cu, rem = per % t.per_cu;
+  const float kspan = (float)((K / kTK + splits - 1) / splits);
+  const float us = (float)full * std::max(t.alone, t.per_cu * t.each) * kspan +
+                   (rem ? std::max(t.alone, rem * t.each) * kspan : 0.f) + 3.f * (full + (rem > 0));
+  return us + (splits > 1 ? 3.f + (splits + 1) * (float)(M * N) * 4e-6f / 3.f : 0.f);
+}
+
+struct TiledPlan {
+  TiledShape shape;
+  int splits;
+  float us;  // (up to kShapeRows rows)
+};
+// `splits` > 0: with that many.  Otherwise 1, 2, 4 or 8 of at least 16 k-steps
+// where the call can take several.
+TiledPlan tiled_plan(int64_t M, int64_t N, int64_t K, Epilogue ep, int splits) {
+  // 128 x 256 workgroup tiles (64 x 128 per wave, 2 workgroups per CU) for
+  // wide outputs: per MFMA a third less LDS traffic (copies + fragment
+  // reads) than 128 x 128 tiles at 3 per CU.  Measured at config 4's prefill
+  // shapes: gate/up (N 11264) 649-673 -> 692-700 TFLOP/s; QKV (2560) even,
+  // down (2048) -3 %, O (2048) -13 % (too few tiles for 2 per CU).
+  // ORION_GEMM_WIDE=0/1 forces the choice (measurement knob, read per call).
+  const char* wide_env = getenv("ORION_GEMM_WIDE");
+  const bool can_split = ep != Epilogue::kSwiGLU;
+  if (wide_env || M > kShapeRows) {
+    const bool wide = wide_env ? wide_env[0] == '1' : N >= 8192;
+    const int s = !can_split ? 1 : splits ? splits : tiled_ksplits(M, N, K);
+    return {wide ? kTiledWide : kTiledShapes[0], s, 0.f};
+  }
+  const bool forced = getenv("ORION_GEMM_TILED_SPLIT") != nullptr;
+  if (can_split && !splits && forced) splits = tiled_ksplits(M, N, K);
+  TiledPlan best{kTiledShapes[0], 1, 1e30f};
+  for (const TiledShape& t : kTiledShapes)
+    for (int s = 1; s <= 8; s *= 2) {
+      const int n = !can_split ? 1 : splits ? splits : s;
+      if (n > 1 && !splits && K / kTK / n < 16) break;
+      const float us = tiled_cost(t, M, N, K, n);
+      if (us < best.us) best = {t, n, us};
+      if (n != s) break;
+    }
+  return best;
+}
 }  // namespace
+
+bool gemm_takes_rope(int64_t M, int64_t N, int64_t K, int64_t head_dim) {
+  if (head_dim % 32 != 0) return false;
+  const TiledPlan best = tiled_plan(M, N, K, Epilogue::kStore, 0);
+  if (best.splits == 1 || M > kShapeRows || getenv("ORION_GEMM_TILED_SPLIT")) return best.splits == 1;
+  // unsplit and without RoPE's launch, a read and a write of the matrix
+  const float saved = 3.f + (float)(M * N) * 8e-6f / 3.f;
+  return tiled_plan(M, N, K, Epilogue::kStore, 1).us < best.us + saved;
+}
 
 void gemm_scratch_need(int64_t M, int64_t N, int64_t K, size_t* ws_bytes, bool preferred) {
   *ws_bytes = 0;
   if (M < 1 || K % 32 != 0) return;
   if (M > 64) {
-    const int s = tiled_ksplits(M, N, K, preferred);
+    const int s = preferred ? tiled_plan(M, N, K, Epilogue::kStore, 0).splits
+                            : tiled_ksplits(M, N, K, false);
     if (s > 1) *ws_bytes = (size_t)s * (size_t)M * (size_t)N * sizeof(float);
     return;
   }
@@ -865,16 +1061,26 @@ hipError_t launch_gemm(hipStream_t st, const float* x, const uint16_t* w, const 
       pk.pair_dim = (int)f.pair_dim;
       pk.pair_cols = (int)f.pair_cols;
     }
-    // 128 x 256 workgroup tiles (64 x 128 per wave, 2 workgroups per CU) for
-    // wide outputs: per MFMA a third less LDS traffic (copies + fragment
-    // reads) than 128 x 128 tiles at 3 per CU.  Measured at config 4's prefill
-    // shapes: gate/up (N 11264) 649-673 -> 692-700 TFLOP/s; QKV (2560) even,
-    // down (2048) -3 %, O (2048) -13 % (too few tiles for 2 per CU).
-    // ORION_GEMM_WIDE=0/1 forces the choice (measurement knob, read per call).
-    const char* wide_env = getenv("ORION_GEMM_WIDE");
-    const bool wide = wide_env ? wide_env[0] == '1' : N >= 8192;
-    const int tn = wide ? 2 * kTN : kTN;
-    dim3 grid((unsigned)((N + tn - 1) / tn), (unsigned)((M + kTM - 1) / kTM));
+    // Shape and K splits (tiled_plan), when the scratch holds their sums
+    const size_t avail = scratch ? scratch->ws_bytes : 0;
+    auto fits = [&](int s) {
+      return s == 1 || (size_t)s * (size_t)M * (size_t)N * sizeof(float) <= avail;
+    };
+    TiledPlan plan = tiled_plan(M, N, K, ep, f.rope ? 1 : 0);
+    if (!fits(plan.splits)) plan = tiled_plan(M, N, K, ep, tiled_ksplits(M, N, K, false));
+    if (!fits(plan.splits)) plan = tiled_plan(M, N, K, ep, 1);
+    // ORION_GEMM_ACT=bf16 rounds the activations to bf16 (one MFMA per
+    // fragment) instead of the hi/lo pair (measurement knob, read per call).
+    const char* act = getenv("ORION_GEMM_ACT");
+    const bool hilo = !(act && act[0] == 'b');
+    if (f.x_hilo && !hilo) return hipErrorInvalidValue;
+    if (f.rope && (!f.x_hilo || !pk.packed || ep != Epilogue::kStore || pk.pair_dim % 32 != 0 ||
+                   pk.pair_dim < 32))
+      return hipErrorInvalidValue;
+    if (!hilo && plan.shape.ntw == 4) plan.shape = kTiledShapes[0];
+    const int tn = 32 * plan.shape.ntw, tm = 32 * plan.shape.mtw;
+    int splits = plan.splits;
+    dim3 grid((unsigned)((N + tn - 1) / tn), (unsigned)((M + tm - 1) / tm));
     // XCD-aware grouped tile order with groups of 4 m tiles (measured at the
     // config-4 prefill shapes against the row-major grid: QKV 529 -> 563, O
     // 405 -> 443, down 513 -> 536 TFLOP/s, gate/up unchanged; groups of 8 and
@@ -886,12 +1092,6 @@ hipError_t launch_gemm(hipStream_t st, const float* x, const uint16_t* w, const 
       const int64_t total = (int64_t)grid.x * grid.y;
       grid = dim3((unsigned)(((total + 7) / 8) * 8), 1);
     }
-    // K splits (tiled_ksplits), when the scratch holds their sums
-    const size_t avail = scratch ? scratch->ws_bytes : 0;
-    auto fits = [&](int s) { return (size_t)s * (size_t)M * (size_t)N * sizeof(float) <= avail; };
-    int splits = ep == Epilogue::kSwiGLU ? 1 : tiled_ksplits(M, N, K);
-    if (splits > 1 && !fits(splits)) splits = tiled_ksplits(M, N, K, false);
-    if (splits > 1 && !fits(splits)) splits = 1;
     const int ksteps = (int)(K / kTK), kspan = (ksteps + splits - 1) / splits;
     // every split must start below K: with kspan rounded up, ceil(ksteps /
     // kspan) splits cover K (a forced count such as 16 splits of 66 k-steps
@@ -899,17 +1099,34 @@ hipError_t launch_gemm(hipStream_t st, const float* x, const uint16_t* w, const 
     splits = (ksteps + kspan - 1) / kspan;
     grid.z = (unsigned)splits;
     float* partial = splits > 1 ? scratch->ws : nullptr;
-    // ORION_GEMM_ACT=bf16 rounds the activations to bf16 (one MFMA per
-    // fragment) instead of the hi/lo pair (measurement knob, read per call).
-    const char* act = getenv("ORION_GEMM_ACT");
-    const bool hilo = !(act && act[0] == 'b');
-    if (f.x_hilo && !hilo) return hipErrorInvalidValue;
-    auto kern = f.x_hilo ? (wide ? gemm_tiled_kernel<true, 8, true> : gemm_tiled_kernel<true, 4, true>)
-                : wide   ? (hilo ? gemm_tiled_kernel<true, 8> : gemm_tiled_kernel<false, 8>)
-                         : (hilo ? gemm_tiled_kernel<true, 4> : gemm_tiled_kernel<false, 4>);
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, x, f.w_packed ? f.w_packed : w, bias,
-                       (int)M, (int)N, (int)K, (int)ep, out, pk, gm, kspan, partial,
-                       f.out_hilo && ep == Epilogue::kSwiGLU);
+    auto launch = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, x, f.w_packed ? f.w_packed : w, bias,
+                         (int)M, (int)N, (int)K, (int)ep, out, pk, gm, kspan, partial,
+                         f.out_hilo && ep == Epilogue::kSwiGLU, f.rope ? *f.rope : RopeOut{});
+      return hipGetLastError();
+    };
+    auto hilo_shape = [&](auto xs, auto rope) {
+      constexpr bool X = decltype(xs)::value, R = decltype(rope)::value;
+      const TiledShape& t = plan.shape;
+      if (t.ntw == 8) return launch(gemm_tiled_kernel<true, 8, X, 4, 2, R>);
+      switch (t.mtw * 10 + t.st) {
+        case 24: return launch(gemm_tiled_kernel<true, 4, X, 2, 4, R>);
+        case 32: return launch(gemm_tiled_kernel<true, 4, X, 3, 2, R>);
+        case 33: return launch(gemm_tiled_kernel<true, 4, X, 3, 3, R>);
+        case 43: return launch(gemm_tiled_kernel<true, 4, X, 4, 3, R>);
+        case 53: return launch(gemm_tiled_kernel<true, 4, X, 5, 3, R>);
+        default: return launch(gemm_tiled_kernel<true, 4, X, 4, 2, R>);
+      }
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
+    const hipError_t err =
+        !hilo ? (plan.shape.ntw == 8 ? launch(gemm_tiled_kernel<false, 8>)
+                                     : launch(gemm_tiled_kernel<false, 4>))
+        : f.rope   ? hilo_shape(Yes{}, Yes{})
+        : f.x_hilo ? hilo_shape(Yes{}, No{})
+                   : hilo_shape(No{}, No{});
+    if (err != hipSuccess) return err;
     if (splits > 1) {
       const int64_t total = M * N;
       const unsigned blocks = (unsigned)std::min<int64_t>((total + 255) / 256, 8192);

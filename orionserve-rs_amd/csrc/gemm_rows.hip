@@ -74,19 +74,6 @@ __device__ inline void rows_epilogue(const RowsGemm& g, int row, int col, float 
   }
 }
 
-__device__ inline void store_kv1(void* base, bool bf16, int64_t at, float v) {
-  if (bf16)
-    static_cast<uint16_t*>(base)[at] = f32_to_bf16(v);
-  else
-    static_cast<float*>(base)[at] = v;
-}
-
-// Where a row's new K/V vector goes, and its position.
-struct RowSlot {
-  int64_t kv;
-  uint32_t pos;
-};
-
 // QKV with RoPE and the cache write: the 16 columns of a Q or K tile are 8 of
 // the head's first half and the 8 they rotate with (packed_column), a V tile
 // 16 consecutive ones.  The same f32 expressions as rope_cache_kernel.
@@ -250,13 +237,7 @@ __global__ void __launch_bounds__(64 * rows_waves(MT, NT, FRAG)) gemm_rows_kerne
     if (nj == 0 && nrow < MT * 16)
       nscale[nrow] = (float)(1.0 / sqrt(t / (double)K + (double)g.norm_eps));
   }
-  if (g.rope.q_out && tid < MT * 16) {
-    const RopeOut& r = g.rope;
-    const int row = min(tid, M - 1);
-    const uint32_t pos = r.positions[row];
-    const uint32_t blk = r.bt_ids[r.bt_off[r.row_seq[row]] + (pos >> r.bs_log2)];
-    slots[tid] = {(int64_t)blk * r.blk + (int64_t)(pos & ((1u << r.bs_log2) - 1)) * r.slot, pos};
-  }
+  if (g.rope.q_out && tid < MT * 16) slots[tid] = row_slot(g.rope, min(tid, M - 1));
   if (n > 0) {
     int s = 0;
     for (; s + U < n; s += U) {

@@ -293,6 +293,24 @@ struct RopeOut {
   const float* cos = nullptr;
   const float* sin = nullptr;
 };
+#ifdef __HIPCC__
+// Where a row's new K/V vector goes, and its position.
+struct RowSlot {
+  int64_t kv;
+  uint32_t pos;
+};
+__device__ inline RowSlot row_slot(const RopeOut& r, int row) {
+  const uint32_t pos = r.positions[row];
+  const uint32_t blk = r.bt_ids[r.bt_off[r.row_seq[row]] + (pos >> r.bs_log2)];
+  return {(int64_t)blk * r.blk + (int64_t)(pos & ((1u << r.bs_log2) - 1)) * r.slot, pos};
+}
+__device__ inline void store_kv1(void* base, bool bf16, int64_t at, float v) {
+  if (bf16)
+    static_cast<uint16_t*>(base)[at] = f32_to_bf16(v);
+  else
+    static_cast<float*>(base)[at] = v;
+}
+#endif
 // A projection of a decode-shaped forward (gemm_rows.hip) on packed weights.
 struct RowsGemm {
   const float* x = nullptr;  // f32 rows, or fragment order (x_frag)
@@ -342,7 +360,13 @@ struct GemmFuse {
   // output is written that way.
   bool x_hilo = false;
   bool out_hilo = false;
+  // QKV: rotate and write the cache and rope->q_out instead of `out`
+  // (gemm_takes_rope; x_hilo)
+  const RopeOut* rope = nullptr;
 };
+// Whether a QKV launch_gemm of this shape should take RoPE and the cache write
+// into its epilogue: it runs unsplit, and a head is whole pairs of 16-column tiles.
+bool gemm_takes_rope(int64_t M, int64_t N, int64_t K, int64_t head_dim);
 
 // Scratch a launch_gemm call of this shape uses: the decode GEMMs' K-slice
 // partials, or the LDS-tiled GEMM's K-split sums (launch_gemm leaves a tiled

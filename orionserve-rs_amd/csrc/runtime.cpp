@@ -1480,7 +1480,7 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   const char* fuse_env = getenv("ORION_GEMM_FUSE");
   const bool rows_route = allow_pack && n <= kRowsMax;
   const bool fused = rows_route && !(fuse_env && fuse_env[0] == '0');
-  const bool fused_rope = fused && m->pair_dim;
+  bool fused_rope = fused && m->pair_dim;
   // activations between the layer's kernels in fragment order
   const bool frag = rows_route && n >= kFragMinRows;
   const bool rows_head = allow_pack && S <= kRowsMax;
@@ -1735,6 +1735,9 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   const char* act_env = getenv("ORION_GEMM_ACT");
   presplit = n > kRowsMax && allow_pack && H % 8 == 0 && F % 8 == 0 &&
              !(presplit_env && presplit_env[0] == '0') && !(act_env && act_env[0] == 'b');
+  // there the QKV GEMM rotates and writes the cache too, where it can
+  if (presplit && m->pair_dim && !(fuse_env && fuse_env[0] == '0'))
+    fused_rope = gemm_takes_rope(n, m->qkvd, H, d.head_dim);
   // (the rows route's embed also leaves the row sums of squares, so layer
   // 0's QKV GEMM applies its RMSNorm like every later layer's)
   HIP_TRY(st, launch_embed(stream, d_tok, n, m->w_embed, H, hidden, rows_route ? sumsq : nullptr,
@@ -1752,6 +1755,25 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   while ((1 << bs_log2) < d.block_size) ++bs_log2;
   for (int64_t l = 0; l < d.num_layers; ++l) {
     const LayerDev& L = m->layers[l];
+    RopeOut rope;
+    if (fused_rope) {
+      rope.q_out = qrot;
+      rope.kv_bf16 = m->kv.dtype_bf16;
+      rope.kv = static_cast<char*>(m->arena) + l * as.layer * (rope.kv_bf16 ? 2 : 4);
+      rope.hq = (int)Hq;
+      rope.hkv = d.num_kv_heads;
+      rope.bs_log2 = bs_log2;
+      rope.blk = as.blk;
+      rope.v_off = as.v_off;
+      rope.slot = as.slot;
+      rope.head = as.head;
+      rope.positions = d_pos;
+      rope.row_seq = d_rs;
+      rope.bt_off = d_btoff;
+      rope.bt_ids = d_btids;
+      rope.cos = m->rope_cos;
+      rope.sin = m->rope_sin;
+    }
     // QKV input: rms_norm(hidden) * input_norm -- inside the QKV GEMM on the
     // rows route, else a kernel of its own.
     if (!rows_route)
@@ -1763,29 +1785,12 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
       g.bias = L.b_qkv;
       g.pair_dim = m->pair_dim;
       g.pair_cols = m->qd + m->kvd;
-      if (fused_rope) {
-        RopeOut& r = g.rope;
-        r.q_out = qrot;
-        r.kv_bf16 = m->kv.dtype_bf16;
-        r.kv = static_cast<char*>(m->arena) + l * as.layer * (r.kv_bf16 ? 2 : 4);
-        r.hq = (int)Hq;
-        r.hkv = d.num_kv_heads;
-        r.bs_log2 = bs_log2;
-        r.blk = as.blk;
-        r.v_off = as.v_off;
-        r.slot = as.slot;
-        r.head = as.head;
-        r.positions = d_pos;
-        r.row_seq = d_rs;
-        r.bt_off = d_btoff;
-        r.bt_ids = d_btids;
-        r.cos = m->rope_cos;
-        r.sin = m->rope_sin;
-      }
+      g.rope = rope;
       HIP_TRY(st, gemm_rows_on(m->dev, g));
     } else {
       GemmFuse f;
       f.x_hilo = presplit;
+      if (fused_rope) f.rope = &rope;
       if (allow_pack) f.w_packed = L.p_qkv, f.pair_dim = m->pair_dim, f.pair_cols = m->qd + m->kvd;
       HIP_TRY(st, gemm_on(m->dev, xn, L.w_qkv, L.b_qkv, n, m->qkvd, H, Epilogue::kStore, qkv, &f));
     }
