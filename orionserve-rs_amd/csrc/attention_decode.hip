@@ -637,7 +637,7 @@ __device__ inline void group_merge(const float* parts, int stride, int n, int ro
       l += w * p[G * D + 2 * g + 1];
       v += w * p[i];
     }
-    v *= 1.f / l;
+    v = v / l;
     if (out.frag)
       store_frag(out.frag, out.mtiles, row, (kvh * G + g) * D + d, v);
     else

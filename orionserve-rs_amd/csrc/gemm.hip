@@ -933,12 +933,12 @@ int tiled_ksplits(int64_t M, int64_t N, int64_t K, bool preferred = true) {
 // its k-steps in a row times what one costs: `alone` us where the CU holds one
 // workgroup (latency; with two k-steps in LDS one copy is in flight, and it
 // is waited for) or `each` us per resident one where they fill the matrix cores.
-// Measured at 65 to 743 rows of N 4096, 6144 and 28672, K 4096 and 14336; the
-// estimate from these was within 15 % of each time.  160 rows, us before (128
-// rows and two k-steps in LDS; 256 columns at N 28672) and now: QKV 6144 x 4096
-// 38 -> 31, O 4096 x 4096 36 -> 25, gate/up 28672 x 4096 133 -> 85, down 4096 x
-// 14336 62 -> 48; 743 rows: QKV 105 -> 72, O 67 -> 56, gate/up 273 -> 240, down
-// 155 -> 140.
+// Over 65 to 743 rows of N 4096, 6144 and 28672, K 4096 and 14336, in 1 to 8
+// splits, the estimate was within 25 % of 98 in 100 times, and what it chooses
+// 2 % slower than the fastest on average, 13 % at most.  160 rows, us before
+// (128 rows and two k-steps in LDS; 256 columns at N 28672) and now: QKV 6144 x
+// 4096 38 -> 31, O 4096 x 4096 36 -> 25, gate/up 28672 x 4096 133 -> 86, down
+// 4096 x 14336 62 -> 48; 743 rows: QKV 105 -> 72, O 67 -> 60, gate/up 273 -> 240.
 struct TiledShape {
   int ntw, mtw, st, per_cu;
   float alone, each;
