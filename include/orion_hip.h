@@ -319,7 +319,11 @@ int orion_hip_model_kv_layout(orion_hip_model* model, orion_hip_kv_layout* out);
  * prefix caching leaves them) attend that prefix together on bf16 arenas at
  * head_dim 64/128: the query heads of up to 16 / (query heads per KV head)
  * such rows share one work item per prefix piece ("packed" items), so each
- * prefix block is read once per pack rather than once per row. */
+ * prefix block is read once per pack rather than once per row.
+ * Few rows of short contexts that share no block run as one workgroup per
+ * (row, KV head), which merges its waves' pieces itself: no merge launch
+ * follows, and the counts of orion_hip_decode_plan_info are those of the
+ * separate items it replaces. */
 typedef struct orion_hip_decode_plan orion_hip_decode_plan;
 int orion_hip_decode_plan_create(orion_hip_device* dev, const uint32_t* positions,
                                  const int32_t* row_seq, const int64_t* block_table_offsets,
