@@ -391,19 +391,18 @@ int decode_group_waves(const KvGeom& kv, int64_t hq) {
   return kv.head_dim == 64 ? kGroupWaves[G <= 4] : 0;
 }
 
-// Longest piece of a grouped row: two 16-token steps, or four where bf16 rows
-// are at most a pair per four CUs (the f32 wave holds two).  Against separate
-// items and merge, one row of up to 500 tokens took 5.3 us for 8.7 (bf16,
-// head_dim 64, 4 KV heads) and 6.3 for 10.9 (f32), 32 rows of them 7.4 for 8.5,
-// and 4 rows of up to 500 at head_dim 128, 8 KV heads, 8.7 for 9.5.  With four
-// steps a wave for more pairs, 32 rows of up to 1000 tokens took 10.1 us for 9.9
-// and a 22-layer step of them 1607 for 1567: there the pieces over all CUs are
-// worth the merge launch, as they are with more (row, KV head) pairs than CUs.
+// Longest piece of a grouped row: two 16-token steps.  Against separate items
+// and merge, one row of up to 500 tokens took 5.3 us for 8.7 (bf16, head_dim 64,
+// 4 KV heads) and 6.3 for 10.9 (f32), 32 rows of them 7.4 for 8.5.  Four steps a
+// wave lost: 32 rows of up to 1000 tokens took 10.1 us for 9.9, a 22-layer step of
+// them 1607 for 1567, and one of a single row of 700 tokens, whose K and V are not
+// in a cache, 1053 for 1039.  There the pieces over all CUs are worth the merge
+// launch, as they are with more (row, KV head) pairs than CUs.
 constexpr int kGroupPiece = 32;
 
 void build_decode_groups(const uint32_t* positions, const int32_t* row_seq,
                          const int64_t* bt_offsets, const uint32_t* bt_ids, int64_t rows,
-                         int64_t hkv, int64_t block_size, int64_t cus, int group_waves, bool bf16,
+                         int64_t hkv, int64_t block_size, int64_t cus, int group_waves,
                          const uint8_t* skip_rows, DecodePlanHost* plan) {
   plan->groups.clear();
   plan->group_waves = 0;
@@ -421,8 +420,7 @@ void build_decode_groups(const uint32_t* positions, const int32_t* row_seq,
     ++planned;
     longest = std::max<int64_t>(longest, (int64_t)positions[r] + 1);
   }
-  const int64_t longest_piece = bf16 && planned * hkv * 4 <= cus ? 2 * kGroupPiece : kGroupPiece;
-  if (planned * hkv > cus || longest > longest_piece * group_waves || unit > longest_piece)
+  if (planned * hkv > cus || longest > (int64_t)kGroupPiece * group_waves || unit > kGroupPiece)
     return;
   plan->group_waves = group_waves;
   plan->groups.reserve((size_t)(planned * hkv * group_waves));

@@ -125,7 +125,7 @@ int decode_group_waves(const KvGeom& kv, int64_t hq);
 // (group_waves of 0 leaves the plan as it is).
 void build_decode_groups(const uint32_t* positions, const int32_t* row_seq,
                          const int64_t* bt_offsets, const uint32_t* bt_ids, int64_t rows,
-                         int64_t hkv, int64_t block_size, int64_t cus, int group_waves, bool bf16,
+                         int64_t hkv, int64_t block_size, int64_t cus, int group_waves,
                          const uint8_t* skip_rows, DecodePlanHost* plan);
 size_t decode_workspace_bytes(int64_t rows, int64_t hq, int64_t D, int64_t max_splits);
 // Rows per packed prefix item for this arena and grouping (0: no packing).

@@ -1590,7 +1590,7 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
                       npf ? skip.data() : nullptr, &plan, decode_pack_rows(m->kv, Hq));
     build_decode_groups(b->positions, hb.row_seq.data(), b->block_table_offsets,
                         b->block_table_ids, n, d.num_kv_heads, d.block_size,
-                        m->dev->wave_slots / 8, decode_group_waves(m->kv, Hq), m->kv.dtype_bf16,
+                        m->dev->wave_slots / 8, decode_group_waves(m->kv, Hq),
                         npf ? skip.data() : nullptr, &plan);
     // One workspace for the decode splits and the prefill key parts (their
     // launches are ordered on the stream: the decode merge has read the
@@ -1939,7 +1939,7 @@ ORION_EXPORT int orion_hip_decode_plan_create(orion_hip_device* dev, const uint3
   auto group = [&](const KvGeom& geom, DecodePlanHost* h) {
     build_decode_groups(positions, row_seq, block_table_offsets, block_table_ids, num_rows,
                         num_kv_heads, block_size, dev->wave_slots / 8,
-                        decode_group_waves(geom, num_q_heads), geom.dtype_bf16, nullptr, h);
+                        decode_group_waves(geom, num_q_heads), nullptr, h);
   };
   group(bf16_geom, &p->host);
   if (p->has_plain()) {

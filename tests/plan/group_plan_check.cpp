@@ -2,10 +2,9 @@
 // orionserve-rs_amd/csrc/decode_plan.cpp), host only.  For random batches a
 // grouped plan must hold group_waves records per planned (row, KV head), in
 // order, whose pieces cover [0, position] exactly once from 16-token-aligned
-// starts, with the row's piece count, at most the longest piece (32 tokens, or 64
-// for a bf16 arena with at most a pair per four CUs), the
+// starts, with the row's piece count, at most 32 tokens, the
 // right table offset and first block, and empty records after them; and the
-// plan must stay ungrouped where a row is longer than that per wave, the
+// plan must stay ungrouped where a row is longer than 32 tokens per wave, the
 // pairs outnumber the CUs, rows share blocks, or nothing is split.  Prints one
 // line per failure and a summary; exit status 1 on any failure.
 #include "kernels.hpp"
@@ -25,8 +24,7 @@ int main(int argc, char** argv) {
   for (int trial = 0; trial < trials; ++trial) {
     const int rows = 1 + rng() % 70, bs = 1 << (rng() % 8), hkv = 1 + rng() % 8;
     const int waves = orion::kGroupWaves[rng() % 2];
-    const bool bf16 = rng() % 2;
-    const int maxctx = trial % 3 == 0 ? 40 : trial % 3 == 1 ? 32 * waves : 64 * waves + 100;
+    const int maxctx = trial % 3 == 0 ? 40 : trial % 3 == 1 ? 32 * waves : 32 * waves + 100;
     std::vector<uint32_t> pos(rows), ids;
     std::vector<int32_t> row_seq(rows);
     std::vector<int64_t> off(rows + 1, 0);
@@ -44,10 +42,9 @@ int main(int argc, char** argv) {
     orion::build_decode_plan(pos.data(), row_seq.data(), off.data(), ids.data(), rows, hkv, bs,
                              2048, skip.data(), &plan, 0);
     orion::build_decode_groups(pos.data(), row_seq.data(), off.data(), ids.data(), rows, hkv, bs,
-                               256, waves, bf16, skip.data(), &plan);
-    const int piece = bf16 && planned * hkv * 4 <= 256 ? 64 : 32;
-    const bool want = plan.max_splits > 1 && plan.stream_kv && planned * hkv <= 256 && longest <= piece * waves &&
-                      bs <= piece;
+                               256, waves, skip.data(), &plan);
+    const bool want = plan.max_splits > 1 && plan.stream_kv && planned * hkv <= 256 && longest <= 32 * waves &&
+                      bs <= 32;
     if ((plan.group_waves != 0) != want) fail(trial, "grouped or not");
     if (!plan.group_waves) continue;
     ++grouped;
@@ -65,7 +62,7 @@ int main(int argc, char** argv) {
           if (w.item != r * hkv + h || w.split != s) fail(trial, "order");
           if (w.end == 0) continue;
           if (n != s || w.start != next || w.start % 16 || w.end <= w.start) fail(trial, "piece");
-          if (w.end - w.start > piece || (w.end - 1) / bs - w.start / bs + 1 > piece)
+          if (w.end - w.start > 32 || (w.end - 1) / bs - w.start / bs + 1 > 32)
             fail(trial, "piece length");
           if (w.tbl_off != off[r] + w.start / bs || w.blk0 != (int32_t)ids[w.tbl_off])
             fail(trial, "table");

@@ -34,8 +34,7 @@ def test_grouped_plans_cover_every_context_once(tmp_path):
 def test_grouped_decode_matches_oracle_and_split(backend, monkeypatch, dtype, G, d, bs, head_major):
     from test_gpu_attention import run_decode
 
-    # 32 tokens a wave, 64 in bf16 (20 pairs)
-    longest = (16 if d == 64 and (dtype == "bf16" or G <= 4) else 8) * (64 if dtype == "bf16" else 32)
+    longest = 512 if d == 64 and (dtype == "bf16" or G <= 4) else 256  # 32 tokens a wave
     ctxs = [longest, 1, 15, 16, 17, 63, 64, 65, longest - 1, longest // 2 + 3]
     case = PagedCase(G * d + bs, ctxs, 2 * G, 2, d, bs, dtype=dtype, pool_factor=1.25,
                      head_major=head_major)
