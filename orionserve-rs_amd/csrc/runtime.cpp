@@ -286,7 +286,10 @@ struct orion_hip_model {
   uint16_t* w_lm = nullptr;  // null when tied
   float* final_norm = nullptr;
   uint16_t* p_head = nullptr;  // LM head (or tied embedding) in packed order
-  bool packs_valid = false;    // packed copies match the row-major weights
+  // Packed copies that match their row-major weights: of the matrices that are
+  // freed once packed (matrices()), and of a tied head (the embedding stays).
+  bool packs_valid = false;
+  bool tied_pack_valid = false;
   bool rowmajor_live = true;   // row-major layer matrices / LM head allocated
   std::vector<LayerDev> layers;
   float* rope_cos = nullptr;
@@ -725,13 +728,25 @@ struct WeightSlot {
 
 static hipError_t ensure_rowmajor(orion_hip_model* m);
 
+// Whether a weight is (part of) one of matrices(): packed, and row-major only
+// while it is written or read.
+static bool packed_matrix(const orion_hip_model* m, int which) {
+  return which == ORION_W_Q || which == ORION_W_K || which == ORION_W_V || which == ORION_W_O ||
+         which == ORION_W_GATE || which == ORION_W_UP || which == ORION_W_DOWN ||
+         (which == ORION_W_LM_HEAD && !m->desc.tied_lm_head);
+}
+
+// A weight is about to change: the packed copy made from it, if there is one,
+// is made again by the next forward.  (Norms, biases and an untied embedding
+// have none; the row-major matrices the others would be made from are freed.)
+static void stale_packs(orion_hip_model* m, int which) {
+  if (packed_matrix(m, which)) m->packs_valid = false;
+  if (which == ORION_W_EMBED) m->tied_pack_valid = false;
+}
+
 static int weight_slot(orion_hip_model* m, int which, int layer, WeightSlot* s) {
   const auto& d = m->desc;
-  const bool matrix = which == ORION_W_LM_HEAD || which == ORION_W_Q || which == ORION_W_K ||
-                      which == ORION_W_V || which == ORION_W_O || which == ORION_W_GATE ||
-                      which == ORION_W_UP || which == ORION_W_DOWN;
-  if (matrix && (which != ORION_W_LM_HEAD || !d.tied_lm_head))
-    HIP_TRY("weight", ensure_rowmajor(m));
+  if (packed_matrix(m, which)) HIP_TRY("weight", ensure_rowmajor(m));
   const int64_t H = d.hidden_size, F = d.intermediate_size, V = d.vocab_size;
   if (which >= ORION_W_INPUT_NORM && (layer < 0 || layer >= d.num_layers))
     return internal("upload_weight", "layer %d out of range (have %d)", layer, d.num_layers);
@@ -789,13 +804,13 @@ ORION_EXPORT int orion_hip_model_upload_weight(orion_hip_model* model, int which
   const char* st = "upload_weight";
   WeightSlot s;
   if (int rc = weight_slot(model, which, layer, &s)) return rc;
-  model->packs_valid = false;
   if ((int64_t)count != s.rows * s.cols)
     return internal(st, "weight %d has %zu elements, expected %lld", which, count,
                     (long long)(s.rows * s.cols));
   if (dtype != ORION_DTYPE_F32 && dtype != ORION_DTYPE_F16 && dtype != ORION_DTYPE_BF16)
     return set_err(ORION_HIP_ERR_BACKEND, st, "unsupported host dtype %d", dtype);
   HIP_TRY(st, hipSetDevice(model->dev->ordinal));
+  stale_packs(model, which);
   // Convert on the host (loader.rs:74-98 widens to f32; device matrices are bf16).
   if (s.bf16) {
     if (dtype == ORION_DTYPE_BF16) return upload_rows(model, s, host, 2, st);
@@ -1134,7 +1149,7 @@ static int init_one(orion_hip_model* m, int which, int layer, uint64_t seed, flo
   const char* st = "init_synthetic";
   WeightSlot s;
   if (int rc = weight_slot(m, which, layer, &s)) return rc;
-  m->packs_valid = false;
+  stale_packs(m, which);
   hipStream_t stream = m->dev->stream;
   const float mul = std_ / kIrwinHallSd;
   const uint64_t key = synthetic_key(seed, which, which >= ORION_W_INPUT_NORM ? layer : -1);
@@ -1380,8 +1395,9 @@ static std::vector<MatrixRef> matrices(orion_hip_model* m) {
   return v;
 }
 
-// Writes the packed copy of every layer matrix and the LM head (allocated on
-// first use) from the row-major weights.
+// Writes the packed copies that are out of date (allocated on first use): every
+// layer matrix and the LM head from the row-major weights, a tied head from the
+// embedding.
 static hipError_t make_packs(orion_hip_model* m) {
   const auto& d = m->desc;
   hipStream_t stream = m->dev->stream;
@@ -1394,16 +1410,19 @@ static hipError_t make_packs(orion_hip_model* m) {
     }
     return launch_pack_weights(stream, *r.rowmajor, r.N, r.K, r.pair_dim, r.pair_cols, *r.packed);
   };
-  if (!m->rowmajor_live) return hipErrorInvalidValue;
-  for (const MatrixRef& r : matrices(m)) {
-    hipError_t e = one(r);
-    if (e != hipSuccess) return e;
+  if (!m->packs_valid) {
+    if (!m->rowmajor_live) return hipErrorInvalidValue;
+    for (const MatrixRef& r : matrices(m)) {
+      hipError_t e = one(r);
+      if (e != hipSuccess) return e;
+    }
+    m->packs_valid = true;
   }
-  if (d.tied_lm_head) {
+  if (d.tied_lm_head && !m->tied_pack_valid) {
     hipError_t e = one({&m->w_embed, &m->p_head, d.vocab_size, d.hidden_size, 0, 0});
     if (e != hipSuccess) return e;
+    m->tied_pack_valid = true;
   }
-  m->packs_valid = true;
   return hipSuccess;
 }
 
@@ -1465,7 +1484,7 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
     return !(v && v[0] == '0');
   }();
   if (allow_pack) {
-    if (!m->packs_valid) HIP_TRY(st, make_packs(m));
+    HIP_TRY(st, make_packs(m));
     HIP_TRY(st, release_rowmajor(m));
   } else {
     HIP_TRY(st, ensure_rowmajor(m));

@@ -555,6 +555,40 @@ def test_weights_are_kept_once_and_read_back_after_packing(backend):
     gm.close()
 
 
+@pytest.mark.parametrize("tied", [False, True])
+def test_one_rewritten_weight_after_packing(backend, tied):
+    # Once the layer matrices are packed and their row-major copies freed, any
+    # one weight can be written again (norms, biases and the embedding have no
+    # packed copy, a tied head's comes from the embedding): the next forward
+    # gives bitwise what a model uploaded with those weights gives.  A refused
+    # upload changes nothing.
+    rng = np.random.default_rng(11 + tied)
+    spec = small_spec(bias=True, tied=tied)
+    W, other = random_weights(spec, rng, std=0.05), random_weights(spec, rng, std=0.05)
+    gm = gpu_model(backend, spec, W, oh.F32)
+    b = batch([1, 2, 3, 4], [0, 1, 2, 3], [4], [[0]])
+    before = gm.forward(b).logits
+    for which, layer, key in [(oh.W_INPUT_NORM, 1, "input_norm"), (oh.W_POST_NORM, 0, "post_norm"),
+                              (oh.W_K_BIAS, 1, "k_bias"), (oh.W_EMBED, -1, "embed"),
+                              (oh.W_FINAL_NORM, -1, "final_norm"), (oh.W_GATE, 0, "gate"),
+                              (oh.W_LM_HEAD, -1, "lm_head")]:
+        if which == oh.W_LM_HEAD and tied:
+            continue
+        at, src = (W, other) if layer < 0 else (W["layers"][layer], other["layers"][layer])
+        with pytest.raises(oh.InternalError):
+            gm.upload_weight(which, layer, src[key].reshape(-1)[:-1])
+        assert np.array_equal(gm.forward(b).logits, before), key
+        gm.upload_weight(which, layer, src[key])
+        at[key] = src[key]
+        got = gm.forward(b).logits
+        fresh = gpu_model(backend, spec, W, oh.F32)
+        assert np.array_equal(got, fresh.forward(b).logits), key
+        fresh.close()
+        assert not np.array_equal(got, before), key
+        before = got
+    gm.close()
+
+
 def test_prepared_batch_forward_is_identical(backend):
     """A batch flattened once (ForwardBatch.prepare) gives bitwise the same
     logits as one flattened per call; the library still validates it."""
