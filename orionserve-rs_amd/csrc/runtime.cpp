@@ -117,6 +117,17 @@ struct PinnedBuf {
   }
 };
 
+// The end of a call that queues work on pinned memory the next call writes or
+// frees: every way out of it waits for the stream, errors included.  Armed by
+// setting the stream before the first such work, disarmed by the call's own
+// synchronisation.
+struct StreamWait {
+  hipStream_t stream = nullptr;
+  ~StreamWait() {
+    if (stream) (void)hipStreamSynchronize(stream);
+  }
+};
+
 // Pinned memory to the device, in stream order.
 hipError_t upload(hipStream_t st, void* dst, const void* pinned, size_t bytes) {
   if (bytes <= kHostCopyMax) return launch_host_copy(st, dst, pinned, bytes);
@@ -1045,8 +1056,8 @@ int sample_on(orion_hip_device* dev, float* d_logits, int64_t rows, int64_t voca
   const int64_t nprev = prev_off[rows];
   if (nprev > 0 && !prev_tok) return internal(st, "null prev_tokens");
   // One staging area: params | offsets | tokens | uniforms, copied up, and the
-  // outputs, which the kernel writes there.  (Each call ends with a stream
-  // sync, so the area is free.)
+  // outputs, which the kernel writes there.  (Each call waits for the stream,
+  // so the area is free.)
   const size_t o_par = 0;
   const size_t o_off = (o_par + rows * sizeof(SampleParams) + 7) & ~(size_t)7;
   const size_t o_tok = o_off + (rows + 1) * 8;
@@ -1066,6 +1077,7 @@ int sample_on(orion_hip_device* dev, float* d_logits, int64_t rows, int64_t voca
   if (nprev) std::memcpy(host + o_tok, prev_tok, nprev * 4);
   std::memcpy(host + o_uni, uniform, rows * 4);
   hipStream_t stream = dev->stream;
+  StreamWait queued{stream};
   char* d = static_cast<char*>(dev->sample_io.ptr);
   HIP_TRY(st, upload(stream, d, host, o_out));
   HIP_TRY(st, launch_sample(stream, d_logits, rows, vocab,
@@ -1075,6 +1087,7 @@ int sample_on(orion_hip_device* dev, float* d_logits, int64_t rows, int64_t voca
                             reinterpret_cast<const float*>(d + o_uni),
                             reinterpret_cast<int32_t*>(host + o_out)));
   HIP_TRY(st, hipStreamSynchronize(stream));
+  queued.stream = nullptr;
   std::memcpy(tokens, host + o_out, rows * 4);
   for (int64_t r = 0; r < rows; ++r)  // a greedy row with no number above -inf
     if (tokens[r] < 0) return internal(st, "row %lld: argmax over empty logits", (long long)r);
@@ -1547,8 +1560,9 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   }
   const int64_t npf = (int64_t)pf_start.size();
 
-  // (Each forward ends with a stream sync, so the previous forward's use of
-  // the staging areas is complete.)
+  // (Each forward waits for the stream however it ends, so the previous one's
+  // use of the staging areas is complete.)
+  StreamWait queued;
 
   // ---- upload the batch: tokens, positions, row sequences, last rows and
   // block tables, one pinned staging area, one copy ----
@@ -1569,6 +1583,7 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
     std::memcpy(hp + o_last, hb.last_rows.data(), S * 4);
     std::memcpy(hp + o_btoff, b->block_table_offsets, (S + 1) * 8);
     std::memcpy(hp + o_btids, b->block_table_ids, nbt * 4);
+    queued.stream = stream;
     HIP_TRY(st, upload(stream, m->b_batch.ptr, hp, total));
   }
   const char* dp = m->b_batch.as<char>();
@@ -1761,14 +1776,8 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   // 0's QKV GEMM applies its RMSNorm like every later layer's)
   HIP_TRY(st, launch_embed(stream, d_tok, n, m->w_embed, H, hidden, rows_route ? sumsq : nullptr,
                            xn_frag, m->layers[0].input_norm));
-  // (a refused batch waits for what it has queued: the staging areas are free
-  // again when the call returns)
-  auto refused = [&](int rc) {
-    (void)hipStreamSynchronize(stream);
-    return rc;
-  };
   if (fused_rope)
-    if (int rc = validate_tables(m, b, hb)) return refused(rc);
+    if (int rc = validate_tables(m, b, hb)) return rc;
   const ArenaStrides as = arena_strides(m->kv);
   int bs_log2 = 0;
   while ((1 << bs_log2) < d.block_size) ++bs_log2;
@@ -1814,7 +1823,7 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
       HIP_TRY(st, gemm_on(m->dev, xn, L.w_qkv, L.b_qkv, n, m->qkvd, H, Epilogue::kStore, qkv, &f));
     }
     if (l == 0)
-      if (int rc = plan_attention()) return refused(rc);
+      if (int rc = plan_attention()) return rc;
     if (!fused_rope)
       HIP_TRY(st, launch_rope_and_cache(stream, m->kv, m->arena, l, n, Hq, qkv, m->qkvd, qrot,
                                         qkv + m->qd, m->qkvd, qkv + m->qd + m->kvd, m->qkvd, d_pos,
@@ -1899,6 +1908,7 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   else if (logits_out)
     HIP_TRY(st, hipMemcpyAsync(logits_out, logits, logit_bytes, hipMemcpyDeviceToHost, stream));
   HIP_TRY(st, hipStreamSynchronize(stream));
+  queued.stream = nullptr;
   if (argmax_out) std::memcpy(argmax_out, h_out, S * 8);
   if (logits_pinned) std::memcpy(logits_out, h_out + o_logits, logit_bytes);
   return ORION_HIP_OK;
