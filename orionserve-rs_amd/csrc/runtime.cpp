@@ -225,43 +225,51 @@ struct orion_hip_decode_plan {
   int64_t rows = 0, hq = 0, hkv = 0, head_dim = 0, block_size = 0;
   // host: the plan as built for a bf16 arena (shared prefixes packed where
   // the MFMA wave takes them); plain: the same rows as an f32 arena takes
-  // them, built when that differs.  Each device buffer holds the work items,
-  // the pieces per row, the pack rows, then the groups.
+  // them, built when that differs.  One device buffer holds the lists of both,
+  // host's from byte 0, plain's from plain_at: a plan costs one allocation and
+  // one copy besides its workspace.
   DecodePlanHost host, plain;
-  DevBuf work, work_plain, ws;
+  size_t plain_at = 0;
+  DevBuf lists, ws;
   ~orion_hip_decode_plan() {
-    work.release();
-    work_plain.release();
+    lists.release();
     ws.release();
   }
-  static DecodePlanDev view_of(const DecodePlanHost& h, const DevBuf& b) {
+  // Byte offsets of a plan's lists: the work items, the pieces per row, the
+  // pack rows, then the groups.
+  struct Layout {
+    size_t work, nsplit, packs, groups, end;
+  };
+  static Layout layout(const DecodePlanHost& h, size_t at) {
+    Layout l;
+    l.work = at;
+    l.nsplit = l.work + h.work.size() * sizeof(DecodeWork);
+    l.packs = l.nsplit + h.row_nsplit.size() * sizeof(int32_t);
+    l.groups = (l.packs + h.pack_rows.size() * sizeof(int32_t) + 15) & ~(size_t)15;
+    l.end = l.groups + h.groups.size() * sizeof(DecodeWork);
+    return l;
+  }
+  // f32 arenas take no packs, and groups of another size
+  bool has_plain() const { return host.num_packed || host.group_waves; }
+  DecodePlanDev view(bool bf16) const {
+    const bool f32_plan = !bf16 && has_plain();
+    const DecodePlanHost& h = f32_plan ? plain : host;
+    const Layout l = layout(h, f32_plan ? plain_at : 0);
+    const char* base = lists.as<const char>();
     DecodePlanDev d;
-    d.work = b.as<const DecodeWork>();
-    const char* base = b.as<const char>();
-    d.row_nsplit = reinterpret_cast<const int32_t*>(base + h.work.size() * sizeof(DecodeWork));
+    d.work = reinterpret_cast<const DecodeWork*>(base + l.work);
+    d.row_nsplit = reinterpret_cast<const int32_t*>(base + l.nsplit);
     d.num_work = (int)h.work.size();
     d.chunk = h.chunk;
     d.max_splits = h.max_splits;
     d.stream_kv = h.stream_kv;
     d.mixed_kv = h.mixed_kv;
     d.num_packed = h.num_packed;
-    d.pack_rows = reinterpret_cast<const int32_t*>(base + h.work.size() * sizeof(DecodeWork) +
-                                                   h.row_nsplit.size() * sizeof(int32_t));
+    d.pack_rows = reinterpret_cast<const int32_t*>(base + l.packs);
     d.pack_r = h.pack_r;
-    d.groups = reinterpret_cast<const DecodeWork*>(base + groups_at(h));
+    d.groups = reinterpret_cast<const DecodeWork*>(base + l.groups);
     d.group_waves = h.group_waves;
     d.num_groups = h.group_waves ? (int)(h.groups.size() / h.group_waves) : 0;
-    return d;
-  }
-  // Byte offset of the groups, after the pack rows.
-  static size_t groups_at(const DecodePlanHost& h) {
-    return (h.work.size() * sizeof(DecodeWork) + h.row_nsplit.size() * 4 + h.pack_rows.size() * 4 +
-            15) & ~(size_t)15;
-  }
-  // f32 arenas take no packs, and groups of another size
-  bool has_plain() const { return host.num_packed || host.group_waves; }
-  DecodePlanDev view(bool bf16) const {
-    DecodePlanDev d = (!bf16 && has_plain()) ? view_of(plain, work_plain) : view_of(host, work);
     d.ws = ws.as<float>();
     d.ws_bytes = ws.bytes;
     return d;
@@ -1632,9 +1640,12 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
     HIP_TRY(st, m->ws.reserve(std::max(decode_workspace_bytes(n, Hq, d.head_dim, plan.max_splits),
                                        decode_workspace_bytes(n, Hq, d.head_dim, pfp.max_parts))));
     const std::vector<PrefillTile>& pf_order = pfp.order;
+    // (the items that a grouped plan replaces are not run: they stay here)
+    const size_t work_bytes = plan.group_waves ? 0 : plan.work.size() * sizeof(DecodeWork);
+    const size_t nsplit_bytes = plan.group_waves ? 0 : plan.row_nsplit.size() * 4;
     const size_t o_work = 0;
-    const size_t o_nsplit = o_work + plan.work.size() * sizeof(DecodeWork);
-    const size_t o_pfoff = (o_nsplit + plan.row_nsplit.size() * 4 + 7) & ~(size_t)7;
+    const size_t o_nsplit = o_work + work_bytes;
+    const size_t o_pfoff = (o_nsplit + nsplit_bytes + 7) & ~(size_t)7;
     const size_t o_pfstart = o_pfoff + npf * 8;
     const size_t o_pfcount = o_pfstart + npf * 4;
     const size_t o_pfpos = o_pfcount + npf * 4;
@@ -1648,8 +1659,8 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
     HIP_TRY(st, m->h_plan.reserve(ptotal));
     HIP_TRY(st, m->b_plan.reserve(ptotal));
     char* hp = static_cast<char*>(m->h_plan.ptr);
-    std::memcpy(hp + o_work, plan.work.data(), plan.work.size() * sizeof(DecodeWork));
-    std::memcpy(hp + o_nsplit, plan.row_nsplit.data(), plan.row_nsplit.size() * 4);
+    std::memcpy(hp + o_work, plan.work.data(), work_bytes);
+    std::memcpy(hp + o_nsplit, plan.row_nsplit.data(), nsplit_bytes);
     std::memcpy(hp + o_pfoff, pf_btoff.data(), npf * 8);
     std::memcpy(hp + o_pfstart, pf_start.data(), npf * 4);
     std::memcpy(hp + o_pfcount, pf_count.data(), npf * 4);
@@ -1972,31 +1983,31 @@ ORION_EXPORT int orion_hip_decode_plan_create(orion_hip_device* dev, const uint3
   };
   group(bf16_geom, &p->host);
   if (p->has_plain()) {
-    build_decode_plan(positions, row_seq, block_table_offsets, block_table_ids, num_rows,
-                      num_kv_heads, block_size, dev->wave_slots, nullptr, &p->plain, 0);
+    if (p->host.num_packed)
+      build_decode_plan(positions, row_seq, block_table_offsets, block_table_ids, num_rows,
+                        num_kv_heads, block_size, dev->wave_slots, nullptr, &p->plain, 0);
+    else
+      p->plain = p->host;  // the same items: only the groups differ
     group(f32_geom, &p->plain);
   }
-  // work items, then the pieces per row, then the pack rows, in one buffer
-  auto upload = [&](const DecodePlanHost& h, DevBuf& buf) -> hipError_t {
-    const size_t wbytes = h.work.size() * sizeof(DecodeWork);
-    const size_t nbytes = h.row_nsplit.size() * sizeof(int32_t);
-    const size_t pbytes = h.pack_rows.size() * sizeof(int32_t);
-    const size_t o_groups = orion_hip_decode_plan::groups_at(h);
-    const size_t total = o_groups + h.groups.size() * sizeof(DecodeWork);
-    hipError_t e = buf.reserve(total);
-    if (e != hipSuccess) return e;
-    std::vector<char> staged(total);
-    std::memcpy(staged.data(), h.work.data(), wbytes);
-    std::memcpy(staged.data() + wbytes, h.row_nsplit.data(), nbytes);
-    std::memcpy(staged.data() + wbytes + nbytes, h.pack_rows.data(), pbytes);
-    std::memcpy(staged.data() + o_groups, h.groups.data(), h.groups.size() * sizeof(DecodeWork));
-    if (staged.empty()) return hipSuccess;
-    e = hipMemcpyAsync(buf.ptr, staged.data(), staged.size(), hipMemcpyHostToDevice, dev->stream);
-    if (e != hipSuccess) return e;
-    return hipStreamSynchronize(dev->stream);  // staged is freed on return
+  using Layout = orion_hip_decode_plan::Layout;
+  const Layout hl = p->layout(p->host, 0);
+  p->plain_at = (hl.end + 15) & ~(size_t)15;
+  const Layout pl = p->layout(p->plain, p->plain_at);
+  std::vector<char> staged(p->has_plain() ? pl.end : hl.end);
+  auto stage = [&](const DecodePlanHost& h, const Layout& l) {
+    std::memcpy(staged.data() + l.work, h.work.data(), l.nsplit - l.work);
+    std::memcpy(staged.data() + l.nsplit, h.row_nsplit.data(), l.packs - l.nsplit);
+    std::memcpy(staged.data() + l.packs, h.pack_rows.data(), h.pack_rows.size() * 4);
+    std::memcpy(staged.data() + l.groups, h.groups.data(), l.end - l.groups);
   };
-  HIP_TRY(st, upload(p->host, p->work));
-  if (p->has_plain()) HIP_TRY(st, upload(p->plain, p->work_plain));
+  stage(p->host, hl);
+  if (p->has_plain()) stage(p->plain, pl);
+  if (!staged.empty()) {
+    HIP_TRY(st, p->lists.reserve(staged.size()));
+    HIP_TRY(st, hipMemcpyAsync(p->lists.ptr, staged.data(), staged.size(), hipMemcpyHostToDevice,
+                               dev->stream));
+  }
   HIP_TRY(st, p->ws.reserve(decode_workspace_bytes(
                   num_rows, num_q_heads, head_dim,
                   std::max(p->host.max_splits, p->plain.max_splits))));
