@@ -928,7 +928,8 @@ int tiled_ksplits(int64_t M, int64_t N, int64_t K, bool preferred = true) {
 }
 
 // Workgroup tiles of the LDS-tiled GEMM: 32 mtw rows x 32 ntw columns, st
-// k-steps in LDS, `per_cu` workgroups resident (LDS and registers).  Up to
+// k-steps in LDS, `per_cu` workgroups resident (LDS and registers; the form with
+// RoPE also holds its rows' slots, tiled_resident).  Up to
 // kShapeRows rows the grid is a few workgroups per CU, and what a GEMM takes is
 // its k-steps in a row times what one costs: `alone` us where the CU holds one
 // workgroup (latency; with two k-steps in LDS one copy is in flight, and it
@@ -950,14 +951,31 @@ constexpr TiledShape kTiledShapes[] = {
 constexpr TiledShape kTiledWide = {8, 4, 2, 2, 0.f, 0.f};
 constexpr int64_t kShapeRows = 1024;
 constexpr int kCus = 256;
+constexpr int kLdsBytes = 160 * 1024;
 
-// Microseconds of a GEMM on shape t in `splits` K splits: rounds of per_cu
+// Workgroups of shape t that a CU holds.
+constexpr int tiled_resident(const TiledShape& t, bool rope) {
+  const int lds = t.st * (32 * t.mtw * kTK * 4 + 32 * t.ntw * kTK * 2) +
+                  (rope ? 32 * t.mtw * (int)sizeof(RowSlot) : 0);
+  return std::min(t.per_cu, kLdsBytes / lds);
+}
+constexpr bool lds_holds_per_cu() {
+  for (const TiledShape& t : kTiledShapes)
+    if (tiled_resident(t, false) != t.per_cu) return false;
+  return tiled_resident(kTiledWide, false) == kTiledWide.per_cu;
+}
+static_assert(lds_holds_per_cu(), "the table's workgroups per CU fit its LDS");
+// 96 rows x 2 k-steps fill the LDS exactly; with the slots one less fits
+static_assert(tiled_resident(kTiledShapes[2], true) == 3, "four without the slots");
+
+// Microseconds of a GEMM on shape t in `splits` K splits: rounds of resident
 // workgroups, each with a start and an end, and the sums' round trip and launch.
-float tiled_cost(const TiledShape& t, int64_t M, int64_t N, int64_t K, int splits) {
+float tiled_cost(const TiledShape& t, int64_t M, int64_t N, int64_t K, int splits, bool rope) {
+  const int per_cu = tiled_resident(t, rope);
   const int64_t wgs = ((M + 32 * t.mtw - 1) / (32 * t.mtw)) * ((N + 32 * t.ntw - 1) / (32 * t.ntw)) * splits;
-  const int64_t per = (wgs + kCus - 1) / kCus, full = per / t.per_cu, rem = per % t.per_cu;
+  const int64_t per = (wgs + kCus - 1) / kCus, full = per / per_cu, rem = per % per_cu;
   const float kspan = (float)((K / kTK + splits - 1) / splits);
-  const float us = (float)full * std::max(t.alone, t.per_cu * t.each) * kspan +
+  const float us = (float)full * std::max(t.alone, per_cu * t.each) * kspan +
                    (rem ? std::max(t.alone, rem * t.each) * kspan : 0.f) + 3.f * (full + (rem > 0));
   return us + (splits > 1 ? 3.f + (splits + 1) * (float)(M * N) * 4e-6f / 3.f : 0.f);
 }
@@ -968,8 +986,8 @@ struct TiledPlan {
   float us;  // (up to kShapeRows rows)
 };
 // `splits` > 0: with that many.  Otherwise 1, 2, 4 or 8 of at least 16 k-steps
-// where the call can take several.
-TiledPlan tiled_plan(int64_t M, int64_t N, int64_t K, Epilogue ep, int splits) {
+// where the call can take several.  `rope`: the QKV GEMM with RoPE, one split.
+TiledPlan tiled_plan(int64_t M, int64_t N, int64_t K, Epilogue ep, int splits, bool rope = false) {
   // 128 x 256 workgroup tiles (64 x 128 per wave, 2 workgroups per CU) for
   // wide outputs: per MFMA a third less LDS traffic (copies + fragment
   // reads) than 128 x 128 tiles at 3 per CU.  Measured at config 4's prefill
@@ -990,7 +1008,7 @@ TiledPlan tiled_plan(int64_t M, int64_t N, int64_t K, Epilogue ep, int splits) {
     for (int s = 1; s <= 8; s *= 2) {
       const int n = !can_split ? 1 : splits ? splits : s;
       if (n > 1 && !splits && K / kTK / n < 16) break;
-      const float us = tiled_cost(t, M, N, K, n);
+      const float us = tiled_cost(t, M, N, K, n, rope);
       if (us < best.us) best = {t, n, us};
       if (n != s) break;
     }
@@ -1004,7 +1022,7 @@ bool gemm_takes_rope(int64_t M, int64_t N, int64_t K, int64_t head_dim) {
   if (best.splits == 1 || M > kShapeRows || getenv("ORION_GEMM_TILED_SPLIT")) return best.splits == 1;
   // unsplit and without RoPE's launch, a read and a write of the matrix
   const float saved = 3.f + (float)(M * N) * 8e-6f / 3.f;
-  return tiled_plan(M, N, K, Epilogue::kStore, 1).us < best.us + saved;
+  return tiled_plan(M, N, K, Epilogue::kStore, 1, true).us < best.us + saved;
 }
 
 void gemm_scratch_need(int64_t M, int64_t N, int64_t K, size_t* ws_bytes, bool preferred) {
@@ -1066,7 +1084,7 @@ hipError_t launch_gemm(hipStream_t st, const float* x, const uint16_t* w, const 
     auto fits = [&](int s) {
       return s == 1 || (size_t)s * (size_t)M * (size_t)N * sizeof(float) <= avail;
     };
-    TiledPlan plan = tiled_plan(M, N, K, ep, f.rope ? 1 : 0);
+    TiledPlan plan = tiled_plan(M, N, K, ep, f.rope ? 1 : 0, f.rope != nullptr);
     if (!fits(plan.splits)) plan = tiled_plan(M, N, K, ep, tiled_ksplits(M, N, K, false));
     if (!fits(plan.splits)) plan = tiled_plan(M, N, K, ep, 1);
     // ORION_GEMM_ACT=bf16 rounds the activations to bf16 (one MFMA per
