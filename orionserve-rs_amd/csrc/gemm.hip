@@ -417,17 +417,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
     __syncthreads();
   }
   int buf = 0;
-  for (int ks = ks_begin; ks < ksteps; ++ks) {
-    if constexpr (ST > 2) {
-      if (ks + ST - 2 < ksteps)
-        wait_vmem<(ST - 2) * (MTW + BJ)>();
-      else
-        wait_vmem_all();
-      __syncthreads();
-      if (ks + ST - 1 < ksteps) load_tile(ks + ST - 1, buf ? buf - 1 : ST - 1);
-    } else if (ks + 1 < ksteps) {
-      load_tile(ks + 1, buf ^ 1);
-    }
+  auto compute = [&] {
     const uint32_t aoff = (uint32_t)(buf * TM * kTK * 4);
     const uint32_t boff = (uint32_t)(buf * TN * kTK * 2);
     bf16x8 bw[NTW];
@@ -464,12 +454,42 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
               __builtin_amdgcn_mfma_f32_16x16x32_bf16(alo, bw[nt], acc[mt][nt], 0, 0, 0);
       }
     }
-    if constexpr (ST > 2) {
-      buf = buf + 1 < ST ? buf + 1 : 0;
-    } else {
+  };
+  if constexpr (NTW == 8) {
+    // The last k-step apart: a copy in every round of the loop and no branch in
+    // it.  With the stores below, f32 activations, us: 16384 columns x 2048, 400
+    // rows 99 -> 81, 4096 rows 548 -> 490; 32000 x 2048, 4096 rows 1001 -> 905;
+    // 37888 x 3584, 4096 rows 1902 -> 1795.  (128-column tiles at three workgroups
+    // per CU lose 4 to 8 % by it past 1000 rows.)
+    static_assert(ST == 2, "two k-steps in LDS");
+    for (int ks = ks_begin; ks + 1 < ksteps; ++ks) {
+      load_tile(ks + 1, buf ^ 1);
+      compute();
       wait_vmem_all();
       __syncthreads();
       buf ^= 1;
+    }
+    compute();
+  } else {
+    for (int ks = ks_begin; ks < ksteps; ++ks) {
+      if constexpr (ST > 2) {
+        if (ks + ST - 2 < ksteps)
+          wait_vmem<(ST - 2) * (MTW + BJ)>();
+        else
+          wait_vmem_all();
+        __syncthreads();
+        if (ks + ST - 1 < ksteps) load_tile(ks + ST - 1, buf ? buf - 1 : ST - 1);
+      } else if (ks + 1 < ksteps) {
+        load_tile(ks + 1, buf ^ 1);
+      }
+      compute();
+      if constexpr (ST > 2) {
+        buf = buf + 1 < ST ? buf + 1 : 0;
+      } else {
+        wait_vmem_all();
+        __syncthreads();
+        buf ^= 1;
+      }
     }
   }
 
@@ -496,18 +516,49 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NTW ==
     return;
   }
   if (ep == (int)Epilogue::kStore) {
+    if constexpr (NTW == 8) {
+      // A row's columns one after another, and whole tiles without a test per
+      // element: a lane of a 256-column tile stores 128 values.
+      int oc[NTW];
+      float b[NTW];
 #pragma unroll
-    for (int nt = 0; nt < NTW; ++nt) {
-      const int col = n0 + wn * 16 * NTW + nt * 16 + l16;
-      const int oc = packed_column(col, pk.pair_dim, pk.pair_cols);
-      const float b = bias && col < N ? bias[oc] : 0.f;
+      for (int nt = 0; nt < NTW; ++nt) {
+        const int col = n0 + wn * 16 * NTW + nt * 16 + l16;
+        oc[nt] = packed_column(col, pk.pair_dim, pk.pair_cols);
+        b[nt] = bias && col < N ? bias[oc[nt]] : 0.f;
+      }
+      const bool whole = m0 + TM <= M && n0 + TN <= N;
 #pragma unroll
       for (int mt = 0; mt < MTW; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int row = m0 + wm * 16 * MTW + mt * 16 + 4 * grp + i;
-          if (row < M && col < N) out[(int64_t)row * N + oc] = bias ? acc[mt][nt][i] + b : acc[mt][nt][i];
+          float* to = out + (int64_t)row * N;
+          if (whole) {
+#pragma unroll
+            for (int nt = 0; nt < NTW; ++nt)
+              to[oc[nt]] = bias ? acc[mt][nt][i] + b[nt] : acc[mt][nt][i];
+          } else if (row < M) {
+#pragma unroll
+            for (int nt = 0; nt < NTW; ++nt)
+              if (n0 + wn * 16 * NTW + nt * 16 + l16 < N)
+                to[oc[nt]] = bias ? acc[mt][nt][i] + b[nt] : acc[mt][nt][i];
+          }
         }
+    } else {
+#pragma unroll
+      for (int nt = 0; nt < NTW; ++nt) {
+        const int col = n0 + wn * 16 * NTW + nt * 16 + l16;
+        const int oc = packed_column(col, pk.pair_dim, pk.pair_cols);
+        const float b = bias && col < N ? bias[oc] : 0.f;
+#pragma unroll
+        for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int row = m0 + wm * 16 * MTW + mt * 16 + 4 * grp + i;
+            if (row < M && col < N) out[(int64_t)row * N + oc] = bias ? acc[mt][nt][i] + b : acc[mt][nt][i];
+          }
+      }
     }
     return;
   }

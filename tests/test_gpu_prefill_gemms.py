@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
     (256, 8200, 96), (256, 28672, 32), (257, 16384, 64), (320, 24576, 96), (321, 520, 2080),
     (384, 6144, 1056), (480, 136, 4096), (576, 28688, 64), (743, 6152, 512), (768, 4096, 160),
-    (961, 40, 32), (1024, 9216, 96), (1025, 9216, 96)])
+    (961, 40, 32), (1024, 9216, 96), (1025, 9216, 96), (1300, 8200, 64)])
 def test_tiled_shapes_match_linear(backend, M, N, K):
     for kw in (dict(bias=True), dict(accumulate=True)):
         got, _, ref64 = gemm_case(backend, M, N, K, seed=M + N, **kw)
@@ -31,7 +31,9 @@ def test_tiled_shapes_match_linear(backend, M, N, K):
     (160, 96, 14336, 8, 4, 32, oh.F32), (161, 2048, 512, 4, 2, 64, oh.F32),
     (193, 128, 160, 3, 1, 96, oh.F32), (257, 256, 352, 4, 2, 80, oh.F32),
     (320, 64, 7168, 16, 16, 64, oh.F32), (640, 160, 2048, 5, 5, 32, oh.BF16),
-    (1030, 128, 4160, 4, 1, 128, oh.F32)])
+    (1030, 128, 4160, 4, 1, 128, oh.F32),
+    # 8192 QKV columns: 256-column tiles, with RoPE and with the permuted store
+    (1030, 64, 160, 64, 32, 64, oh.F32)])
 def test_prefill_rows_match_oracle_and_separate_rope(backend, monkeypatch, n, H, F, hq, hkv, d, kv):
     rng = np.random.default_rng(n * H + F)
     lens = [n // 2, 3, n - n // 2 - 3]  # ragged prompts, one below a row tile
