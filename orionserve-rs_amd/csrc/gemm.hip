@@ -984,22 +984,30 @@ int tiled_ksplits(int64_t M, int64_t N, int64_t K, bool preferred = true) {
 // kShapeRows rows the grid is a few workgroups per CU, and what a GEMM takes is
 // its k-steps in a row times what one costs: `alone` us where the CU holds one
 // workgroup (latency; with two k-steps in LDS one copy is in flight, and it
-// is waited for) or `each` us per resident one where they fill the matrix cores.
-// Over 65 to 743 rows of N 4096, 6144 and 28672, K 4096 and 14336, in 1 to 8
-// splits, the estimate was within 25 % of 98 in 100 times, and what it chooses
-// 2 % slower than the fastest on average, 13 % at most.  160 rows, us before
-// (128 rows and two k-steps in LDS; 256 columns at N 28672) and now: QKV 6144 x
-// 4096 38 -> 31, O 4096 x 4096 36 -> 25, gate/up 28672 x 4096 133 -> 86, down
-// 4096 x 14336 62 -> 48; 743 rows: QKV 105 -> 72, O 67 -> 60, gate/up 273 -> 240.
+// is waited for) or `each` us per resident one where they fill the matrix cores;
+// [0] for activations that arrive split, [1] for f32 ones, which the kernel splits.
+// Fitted to every shape in 1 to 8 splits on 16 N x K of layers and heads (520 x
+// 1056 to 37888 x 3584, 65 to 1024 rows), weights not in a cache, as a forward
+// finds them; 14 others (704 x 2080 to 128256 x 4096) were kept to check it.
+// There the estimate is within 10 % of 92 in 100 of the times that matter (up to
+// 1.25 x the fastest), and what it chooses is 1.3 % slower than the fastest on
+// average, at most 9 % in 95 of 100.
 struct TiledShape {
   int ntw, mtw, st, per_cu;
-  float alone, each;
+  float alone[2], each[2];
 };
 constexpr TiledShape kTiledShapes[] = {
-    {4, 4, 2, 3, 0.82f, 0.35f}, {4, 4, 3, 2, 0.54f, 0.40f}, {4, 3, 2, 4, 0.77f, 0.275f},
-    {4, 3, 3, 2, 0.47f, 0.335f}, {4, 2, 4, 2, 0.33f, 0.25f}, {4, 5, 3, 1, 0.66f, 0.66f},
+    {4, 4, 2, 3, {0.686f, 0.715f}, {0.431f, 0.512f}},
+    {4, 4, 3, 2, {0.509f, 0.707f}, {0.423f, 0.538f}},
+    {4, 3, 2, 4, {0.728f, 0.623f}, {0.317f, 0.397f}},
+    {4, 3, 3, 2, {0.428f, 0.589f}, {0.332f, 0.445f}},
+    {4, 2, 4, 2, {0.293f, 0.398f}, {0.247f, 0.305f}},
+    {4, 5, 3, 1, {0.620f, 0.895f}, {0.675f, 0.962f}},
+    {8, 4, 2, 2, {0.910f, 1.092f}, {0.782f, 0.885f}},
 };
-constexpr TiledShape kTiledWide = {8, 4, 2, 2, 0.f, 0.f};
+// the shape that batches past kShapeRows rows take, by their columns
+constexpr const TiledShape& kTiledUsual = kTiledShapes[0];
+constexpr const TiledShape& kTiledWide = kTiledShapes[6];
 constexpr int64_t kShapeRows = 1024;
 constexpr int kCus = 256;
 constexpr int kLdsBytes = 160 * 1024;
@@ -1013,22 +1021,27 @@ constexpr int tiled_resident(const TiledShape& t, bool rope) {
 constexpr bool lds_holds_per_cu() {
   for (const TiledShape& t : kTiledShapes)
     if (tiled_resident(t, false) != t.per_cu) return false;
-  return tiled_resident(kTiledWide, false) == kTiledWide.per_cu;
+  return true;
 }
 static_assert(lds_holds_per_cu(), "the table's workgroups per CU fit its LDS");
 // 96 rows x 2 k-steps fill the LDS exactly; with the slots one less fits
 static_assert(tiled_resident(kTiledShapes[2], true) == 3, "four without the slots");
 
 // Microseconds of a GEMM on shape t in `splits` K splits: rounds of resident
-// workgroups, each with a start and an end, and the sums' round trip and launch.
-float tiled_cost(const TiledShape& t, int64_t M, int64_t N, int64_t K, int splits, bool rope) {
+// workgroups (the last of them counts less the fewer CUs have it: the others
+// leave it their share of the L2 and of memory), the launch, and the sums' round
+// trip at 3.9 TB/s.
+float tiled_cost(const TiledShape& t, int64_t M, int64_t N, int64_t K, int splits, bool f32_x,
+                 bool rope) {
   const int per_cu = tiled_resident(t, rope);
+  const float alone = t.alone[f32_x], each = t.each[f32_x];
   const int64_t wgs = ((M + 32 * t.mtw - 1) / (32 * t.mtw)) * ((N + 32 * t.ntw - 1) / (32 * t.ntw)) * splits;
-  const int64_t per = (wgs + kCus - 1) / kCus, full = per / per_cu, rem = per % per_cu;
+  const int64_t per = (wgs + kCus - 1) / kCus, whole = (per - 1) / per_cu;
+  const float idle = (float)(per * kCus - wgs) / kCus, last = (float)(per - whole * per_cu) - 0.3f * idle;
   const float kspan = (float)((K / kTK + splits - 1) / splits);
-  const float us = (float)full * std::max(t.alone, per_cu * t.each) * kspan +
-                   (rem ? std::max(t.alone, rem * t.each) * kspan : 0.f) + 3.f * (full + (rem > 0));
-  return us + (splits > 1 ? 3.f + (splits + 1) * (float)(M * N) * 4e-6f / 3.f : 0.f);
+  const float us = ((float)whole * std::max(alone, per_cu * each) + std::max(alone, last * each)) * kspan +
+                   0.41f * (float)(whole + 1) + 7.1f;
+  return us + (splits > 1 ? (splits + 1) * (float)(M * N) * 4e-6f / 3.9f : 0.f);
 }
 
 struct TiledPlan {
@@ -1037,8 +1050,10 @@ struct TiledPlan {
   float us;  // (up to kShapeRows rows)
 };
 // `splits` > 0: with that many.  Otherwise 1, 2, 4 or 8 of at least 16 k-steps
-// where the call can take several.  `rope`: the QKV GEMM with RoPE, one split.
-TiledPlan tiled_plan(int64_t M, int64_t N, int64_t K, Epilogue ep, int splits, bool rope = false) {
+// where the call can take several.  f32_x: x does not arrive split.  `rope`: the
+// QKV GEMM with RoPE, one split.
+TiledPlan tiled_plan(int64_t M, int64_t N, int64_t K, Epilogue ep, int splits, bool f32_x,
+                     bool rope = false) {
   // 128 x 256 workgroup tiles (64 x 128 per wave, 2 workgroups per CU) for
   // wide outputs: per MFMA a third less LDS traffic (copies + fragment
   // reads) than 128 x 128 tiles at 3 per CU.  Measured at config 4's prefill
@@ -1047,20 +1062,26 @@ TiledPlan tiled_plan(int64_t M, int64_t N, int64_t K, Epilogue ep, int splits, b
   // ORION_GEMM_WIDE=0/1 forces the choice (measurement knob, read per call).
   const char* wide_env = getenv("ORION_GEMM_WIDE");
   const bool can_split = ep != Epilogue::kSwiGLU;
-  if (wide_env || M > kShapeRows) {
-    const bool wide = wide_env ? wide_env[0] == '1' : N >= 8192;
-    const int s = !can_split ? 1 : splits ? splits : tiled_ksplits(M, N, K);
-    return {wide ? kTiledWide : kTiledShapes[0], s, 0.f};
-  }
-  const bool forced = getenv("ORION_GEMM_TILED_SPLIT") != nullptr;
-  if (can_split && !splits && forced) splits = tiled_ksplits(M, N, K);
-  TiledPlan best{kTiledShapes[0], 1, 1e30f};
+  const TiledShape& usual = (wide_env ? wide_env[0] == '1' : N >= 8192) ? kTiledWide : kTiledUsual;
+  const int usual_splits = !can_split ? 1 : splits ? splits : tiled_ksplits(M, N, K);
+  TiledPlan best{usual, usual_splits, 0.f};
+  if (wide_env || M > kShapeRows) return best;
+  if (can_split && !splits && getenv("ORION_GEMM_TILED_SPLIT")) splits = usual_splits;
+  // Up to kShapeRows rows the usual shape stays unless another is estimated 5 %
+  // faster, about what the estimate is off by: of the 1425 calls above 10 are then
+  // more than 3 % slower than on the usual shape (without the margin 36), and all
+  // take 0.82 of its time on average.
+  best.us = tiled_cost(usual, M, N, K, usual_splits, f32_x, rope);
+  float least = 0.95f * best.us;
   for (const TiledShape& t : kTiledShapes)
     for (int s = 1; s <= 8; s *= 2) {
       const int n = !can_split ? 1 : splits ? splits : s;
       if (n > 1 && !splits && K / kTK / n < 16) break;
-      const float us = tiled_cost(t, M, N, K, n, rope);
-      if (us < best.us) best = {t, n, us};
+      const float us = tiled_cost(t, M, N, K, n, f32_x, rope);
+      if (us < least) {
+        best = {t, n, us};
+        least = us;
+      }
       if (n != s) break;
     }
   return best;
@@ -1069,18 +1090,21 @@ TiledPlan tiled_plan(int64_t M, int64_t N, int64_t K, Epilogue ep, int splits, b
 
 bool gemm_takes_rope(int64_t M, int64_t N, int64_t K, int64_t head_dim) {
   if (head_dim % 32 != 0) return false;
-  const TiledPlan best = tiled_plan(M, N, K, Epilogue::kStore, 0);
+  const TiledPlan best = tiled_plan(M, N, K, Epilogue::kStore, 0, false);
   if (best.splits == 1 || M > kShapeRows || getenv("ORION_GEMM_TILED_SPLIT")) return best.splits == 1;
-  // unsplit and without RoPE's launch, a read and a write of the matrix
-  const float saved = 3.f + (float)(M * N) * 8e-6f / 3.f;
-  return tiled_plan(M, N, K, Epilogue::kStore, 1, true).us < best.us + saved;
+  // unsplit, with an epilogue that takes longer, and without RoPE's launch: a read
+  // and a write of the matrix (over 65 to 1024 rows of 2560 x 2048 to 10240 x
+  // 8192, 0.3 % slower on average than always taking the faster of the two)
+  const float saved = 1.f + (float)(M * N) * 8e-6f / 6.f;
+  return tiled_plan(M, N, K, Epilogue::kStore, 1, false, true).us < best.us + saved;
 }
 
-void gemm_scratch_need(int64_t M, int64_t N, int64_t K, size_t* ws_bytes, bool preferred) {
+void gemm_scratch_need(int64_t M, int64_t N, int64_t K, size_t* ws_bytes, bool packed,
+                       bool preferred) {
   *ws_bytes = 0;
   if (M < 1 || K % 32 != 0) return;
   if (M > 64) {
-    const int s = preferred ? tiled_plan(M, N, K, Epilogue::kStore, 0).splits
+    const int s = preferred ? tiled_plan(M, N, K, Epilogue::kStore, 0, !packed).splits
                             : tiled_ksplits(M, N, K, false);
     if (s > 1) *ws_bytes = (size_t)s * (size_t)M * (size_t)N * sizeof(float);
     return;
@@ -1135,9 +1159,13 @@ hipError_t launch_gemm(hipStream_t st, const float* x, const uint16_t* w, const 
     auto fits = [&](int s) {
       return s == 1 || (size_t)s * (size_t)M * (size_t)N * sizeof(float) <= avail;
     };
-    TiledPlan plan = tiled_plan(M, N, K, ep, f.rope ? 1 : 0, f.rope != nullptr);
-    if (!fits(plan.splits)) plan = tiled_plan(M, N, K, ep, tiled_ksplits(M, N, K, false));
-    if (!fits(plan.splits)) plan = tiled_plan(M, N, K, ep, 1);
+    // (a forward's K splits are those of split activations, whichever kernel
+    // splits them: its sums are the same)
+    const bool f32_x = !f.x_hilo;
+    const int want = f.rope || f.unsplit ? 1 : f32_x && pk.packed ? tiled_plan(M, N, K, ep, 0, false).splits : 0;
+    TiledPlan plan = tiled_plan(M, N, K, ep, want, f32_x, f.rope != nullptr);
+    if (!fits(plan.splits)) plan = tiled_plan(M, N, K, ep, tiled_ksplits(M, N, K, false), f32_x);
+    if (!fits(plan.splits)) plan = tiled_plan(M, N, K, ep, 1, f32_x);
     // ORION_GEMM_ACT=bf16 rounds the activations to bf16 (one MFMA per
     // fragment) instead of the hi/lo pair (measurement knob, read per call).
     const char* act = getenv("ORION_GEMM_ACT");
@@ -1146,7 +1174,7 @@ hipError_t launch_gemm(hipStream_t st, const float* x, const uint16_t* w, const 
     if (f.rope && (!f.x_hilo || !pk.packed || ep != Epilogue::kStore || pk.pair_dim % 32 != 0 ||
                    pk.pair_dim < 32))
       return hipErrorInvalidValue;
-    if (!hilo && plan.shape.ntw == 4) plan.shape = kTiledShapes[0];
+    if (!hilo && plan.shape.ntw == 4) plan.shape = kTiledUsual;
     const int tn = 32 * plan.shape.ntw, tm = 32 * plan.shape.mtw;
     int splits = plan.splits;
     dim3 grid((unsigned)((N + tn - 1) / tn), (unsigned)((M + tm - 1) / tm));

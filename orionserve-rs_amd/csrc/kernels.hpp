@@ -363,6 +363,7 @@ struct GemmFuse {
   // QKV: rotate and write the cache and rope->q_out instead of `out`
   // (gemm_takes_rope; x_hilo)
   const RopeOut* rope = nullptr;
+  bool unsplit = false;  // one K split, as with rope
 };
 // Whether a QKV launch_gemm of this shape should take RoPE and the cache write
 // into its epilogue: it runs unsplit, and a head is whole pairs of 16-column tiles.
@@ -373,7 +374,9 @@ bool gemm_takes_rope(int64_t M, int64_t N, int64_t K, int64_t head_dim);
 // GEMM unsplit when the scratch it is given is smaller).
 // preferred: include the optional long-K splits (callers that can grow
 // their scratch); false: only what the call requires.
-void gemm_scratch_need(int64_t M, int64_t N, int64_t K, size_t* ws_bytes, bool preferred = true);
+// packed: GemmFuse::w_packed is set.
+void gemm_scratch_need(int64_t M, int64_t N, int64_t K, size_t* ws_bytes, bool packed,
+                       bool preferred = true);
 hipError_t launch_gemm(hipStream_t st, const float* x, const uint16_t* w, const float* bias,
                        int64_t M, int64_t N, int64_t K, Epilogue ep, float* out,
                        const GemmScratch* scratch = nullptr, const GemmFuse* fuse = nullptr);

@@ -595,10 +595,10 @@ static hipError_t timed_launch(orion_hip_device* dev, int k, F&& launch) {
 }
 
 // The split-K GEMM scratch for a call of this shape, grown on demand.
-static hipError_t gemm_scratch(orion_hip_device* dev, int64_t M, int64_t N, int64_t K,
+static hipError_t gemm_scratch(orion_hip_device* dev, int64_t M, int64_t N, int64_t K, bool packed,
                                GemmScratch* sc) {
   size_t ws = 0;
-  gemm_scratch_need(M, N, K, &ws);
+  gemm_scratch_need(M, N, K, &ws, packed);
   if (ws > dev->gemm_ws.bytes) {
     hipError_t e = dev->gemm_ws.reserve(ws);
     if (e != hipSuccess) return e;
@@ -621,7 +621,7 @@ static hipError_t gemm_on(orion_hip_device* dev, const float* x, const uint16_t*
                           const float* bias, int64_t M, int64_t N, int64_t K, Epilogue ep,
                           float* out, const GemmFuse* fuse = nullptr) {
   GemmScratch sc;
-  hipError_t e = gemm_scratch(dev, M, N, K, &sc);
+  hipError_t e = gemm_scratch(dev, M, N, K, fuse && fuse->w_packed, &sc);
   if (e != hipSuccess) return e;
   return launch_gemm(dev->stream, x, w, bias, M, N, K, ep, out, &sc, fuse);
 }
@@ -1780,9 +1780,11 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
   const char* act_env = getenv("ORION_GEMM_ACT");
   presplit = n > kRowsMax && allow_pack && H % 8 == 0 && F % 8 == 0 &&
              !(presplit_env && presplit_env[0] == '0') && !(act_env && act_env[0] == 'b');
-  // there the QKV GEMM rotates and writes the cache too, where it can
-  if (presplit && m->pair_dim && !(fuse_env && fuse_env[0] == '0'))
-    fused_rope = gemm_takes_rope(n, m->qkvd, H, d.head_dim);
+  // there the QKV GEMM rotates and writes the cache too, where that is worth
+  // running it unsplit (it then is unsplit under every knob: its sums are the same)
+  const bool qkv_unsplit = n > kRowsMax && allow_pack && m->pair_dim &&
+                           gemm_takes_rope(n, m->qkvd, H, d.head_dim);
+  if (presplit && !(fuse_env && fuse_env[0] == '0')) fused_rope = qkv_unsplit;
   // (the rows route's embed also leaves the row sums of squares, so layer
   // 0's QKV GEMM applies its RMSNorm like every later layer's)
   HIP_TRY(st, launch_embed(stream, d_tok, n, m->w_embed, H, hidden, rows_route ? sumsq : nullptr,
@@ -1830,6 +1832,7 @@ ORION_EXPORT int orion_hip_model_forward(orion_hip_model* m, const orion_hip_bat
       GemmFuse f;
       f.x_hilo = presplit;
       if (fused_rope) f.rope = &rope;
+      f.unsplit = qkv_unsplit;
       if (allow_pack) f.w_packed = L.p_qkv, f.pair_dim = m->pair_dim, f.pair_cols = m->qd + m->kvd;
       HIP_TRY(st, gemm_on(m->dev, xn, L.w_qkv, L.b_qkv, n, m->qkvd, H, Epilogue::kStore, qkv, &f));
     }
@@ -2233,7 +2236,7 @@ ORION_EXPORT int orion_hip_gemm_noalloc(orion_hip_device* dev, const float* d_x,
   Epilogue ep;
   if (int rc = gemm_args(st, d_bias, N, K, epilogue, &ep)) return rc;
   size_t need = 0;
-  gemm_scratch_need(M, N, K, &need, false);
+  gemm_scratch_need(M, N, K, &need, false, false);
   if (need > kNoAllocScratchBytes)
     return set_err(ORION_HIP_ERR_BACKEND, st,
                    "M=%lld N=%lld K=%lld needs %zu bytes of split-K scratch; the "

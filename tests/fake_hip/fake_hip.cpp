@@ -2,12 +2,14 @@
 // memory is host memory, copies happen at once, kernels do nothing.  It counts
 // the work queued since the last synchronisation (once pinned memory exists, which
 // that work may read), and makes the n-th call that can fail (an allocation, a
-// copy, a launch) return an error.  Load it with
+// copy, a launch) return an error.  It lists the kernels launched, by name.  Load it with
 // RTLD_GLOBAL before liborion_hip.so, whose HIP calls then come here.
 #include <hip/hip_runtime_api.h>
 
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <string>
 
 namespace {
 int calls = 0, fail_at = 0, queued = 0, pinned = 0, mallocs = 0, copies = 0;
@@ -16,6 +18,8 @@ bool fails() { return ++calls == fail_at; }
 void queue() { queued += pinned > 0; }
 hipError_t error(hipError_t e) { return last = e; }
 char symbol_memory[256];
+std::map<const void*, std::string> kernels;
+std::string launched;
 struct Launch {
   dim3 grid, block;
   size_t shared;
@@ -26,6 +30,8 @@ struct Launch {
 extern "C" {
 void fake_hip_fail_at(int n) { calls = queued = 0, fail_at = n; }
 int fake_hip_calls() { return calls; }
+const char* fake_hip_launched() { return launched.c_str(); }
+void fake_hip_clear_launched() { launched.clear(); }
 int fake_hip_queued() { return queued; }
 int fake_hip_mallocs() { return mallocs; }
 int fake_hip_copies() { return copies; }
@@ -108,8 +114,10 @@ void** __hipRegisterFatBinary(const void*) {
   return &handle;
 }
 void __hipUnregisterFatBinary(void**) {}
-void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*,
-                           void*, int*) {}
+void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*,
+                           void*, void*, int*) {
+  kernels[f] = name;
+}
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t shared, hipStream_t stream) {
   return launch = {grid, block, shared, stream}, hipSuccess;
@@ -119,8 +127,9 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shared,
   *grid = launch.grid, *block = launch.block, *shared = launch.shared, *stream = launch.stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void**, size_t, hipStream_t) {
   if (fails()) return error(hipErrorLaunchFailure);
+  launched += kernels[f] + " " + std::to_string(grid.z) + "\n";
   queue();
   return hipSuccess;
 }
