@@ -22,7 +22,6 @@
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
-#include <type_traits>
 #include <utility>
 
 namespace orion {

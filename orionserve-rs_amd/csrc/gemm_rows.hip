@@ -9,22 +9,23 @@
 // and no reduce launch follows.  The split over workgroups this replaces
 // (slices of 256 k, partials in memory, a reduce launch per GEMM) wrote and
 // read back 16*MT rows of partials per slice: 102 MB at 45 rows x 37888
-// columns x 3584 (271 MB of weights), 150 + 16 us against 63 us here.
+// columns x 3584 (271 MB of weights), 150 + 16 us against 61 us here (4.5 TB/s).
 //
 // What it pays instead is x: every workgroup reads all of it from L2, at about
 // 75 KB/us per CU.  Hence
 //  * the columns per workgroup (rows_shape): as few workgroups as there are
-//    CUs, so each CU reads x once (32 rows x 32000 columns x 2048: 26 us with
-//    250 workgroups of 128 columns, 33 us with 500 of 64, 42 us before);
+//    CUs, so each CU reads x once (32 rows x 32000 columns x 2048, repeated: 26
+//    us with 250 workgroups of 128 columns, 33 us with 500 of 64, 42 us before;
+//    27.8 us in a step, 4.7 TB/s);
 //  * activations in fragment order past 8 rows (kFrag): the producer writes
 //    them split into hi/lo bf16 in the order the lanes read, so a load is one
-//    contiguous KiB and no wave splits (32 rows x 2048 x 2048: 10.4 us from
-//    f32 rows, 7.6 us); up to 8 rows the f32 rows are fewer bytes than 16
-//    padded ones, and stay;
+//    contiguous KiB and no wave splits (32 rows x 2048 x 2048, repeated: 10.4 us
+//    from f32 rows, 7.6 us; 9.5 us in a step); up to 8 rows the f32 rows are
+//    fewer bytes than 16 padded ones, and stay;
 //  * a K split over workgroups where x is far more than a CU's share of W
 //    (rows_shape): partials of few splits and a reduce launch.
 // Weights are read once: their loads are nontemporal, which keeps x in L2
-// (28672 columns x 4096, 32 rows: 51 -> 44 us).
+// (28672 columns x 4096, 32 rows, repeated: 51 -> 44 us).
 #include "common.hpp"
 #include "kernels.hpp"
 

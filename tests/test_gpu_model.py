@@ -387,10 +387,10 @@ def test_tinyllama_shape_greedy_tokens_match_oracle(backend):
 
 @pytest.mark.parametrize("H,F,hq,hkv,d,V", [(160, 224, 2, 1, 64, 1000), (96, 352, 4, 2, 64, 517)])
 def test_odd_shapes_decode_through_packed_weights(backend, H, F, hq, hkv, d, V):
-    # Decode-shaped forwards read the packed weight copies: K that does not
-    # fill a whole K slice (160, 224, 96, 352 over slices of 256) and N that
-    # does not fill a column tile (vocab 1000 and 517 over 128-column tiles)
-    # take the packer's zero padding and the kernel's partial last slice.
+    # Decode-shaped forwards read the packed weight copies: K of fewer k-steps
+    # than a workgroup has waves (160, 224, 96, 352 are 3 to 11 steps of 32), so
+    # that some wave's range is empty, and N that does not fill a column tile
+    # (vocab 1000 and 517 over tiles of 16), which the packer pads with zeros.
     rng = np.random.default_rng(H + F)
     spec = Spec(2, H, hq, hkv, d, F, V, max_pos=512, bias=True, tied=False,
                 num_blocks=48, block_size=16)
@@ -416,23 +416,22 @@ def test_odd_shapes_decode_through_packed_weights(backend, H, F, hq, hkv, d, V):
 
 
 @pytest.mark.parametrize("H,F,hq,hkv,d,V,S,tied,bias", [
-    # hidden > 256 and not a multiple of 256 (partial last K slice in the
-    # norm and sums-of-squares code), vocab not a multiple of 128 (partial
-    # column tile), tied head (the LM head's packed copy comes from the
-    # embedding) with QKV bias (deferred QKV partials + bias in RoPE)
+    # f32 rows, hidden that no count of waves divides evenly, a vocab with a
+    # partial last column tile, a tied head (its packed copy comes from the
+    # embedding) and QKV bias (added in the RoPE epilogue, before the rotation)
     (576, 800, 9, 3, 64, 1000, 5, True, True),
-    # hidden 2304 with 40 rows: more sum-of-squares slots per row than the
-    # early norm path holds, so the GEMMs take the late norm loop
+    # fragment order, and hidden 2304 with 40 rows: 144 sums of squares a row,
+    # more than the 8 per thread that are loaded ahead (the norm's tail loop)
     (2304, 1024, 18, 6, 128, 517, 40, False, False),
 ])
 def test_fused_decode_layer_matches_oracle_and_unfused(backend, monkeypatch, H, F, hq, hkv, d, V,
                                                        S, tied, bias):
-    # Decode batches (one row per sequence, every GEMM split over K) run the
-    # fused layer: RMSNorm applied inside the GEMMs from the residual reduces'
-    # row sums of squares, QKV partials summed by RoPE + cache, and the final
-    # norm inside the LM head.  Checked against the oracle at the f32-KV
-    # bound, and against the same batch with ORION_GEMM_FUSE=0 (separate
-    # norm and reduce launches) at f32 rounding.
+    # Decode batches (one row per sequence, up to 64) run the fused layer:
+    # RMSNorm applied inside the GEMMs from the row sums of squares that the
+    # embedding and the residual GEMMs leave, RoPE and the cache write in the QKV
+    # GEMM's epilogue, and the final norm inside the LM head.  Checked against the
+    # oracle at the f32-KV bound, and against the same batch with
+    # ORION_GEMM_FUSE=0 (norms and RoPE as launches of their own) at f32 rounding.
     rng = np.random.default_rng(H + S)
     spec = Spec(2, H, hq, hkv, d, F, V, max_pos=512, bias=bias, tied=tied,
                 num_blocks=8 * S, block_size=16)
