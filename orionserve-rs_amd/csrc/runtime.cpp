@@ -2006,15 +2006,17 @@ ORION_EXPORT int orion_hip_decode_plan_create(orion_hip_device* dev, const uint3
   };
   stage(p->host, hl);
   if (p->has_plain()) stage(p->plain, pl);
-  if (!staged.empty()) {
-    HIP_TRY(st, p->lists.reserve(staged.size()));
-    HIP_TRY(st, hipMemcpyAsync(p->lists.ptr, staged.data(), staged.size(), hipMemcpyHostToDevice,
-                               dev->stream));
-  }
   HIP_TRY(st, p->ws.reserve(decode_workspace_bytes(
                   num_rows, num_q_heads, head_dim,
                   std::max(p->host.max_splits, p->plain.max_splits))));
-  HIP_TRY(st, hipStreamSynchronize(dev->stream));
+  if (!staged.empty()) {
+    HIP_TRY(st, p->lists.reserve(staged.size()));
+    StreamWait reading{dev->stream};  // staged is freed on return
+    HIP_TRY(st, hipMemcpyAsync(p->lists.ptr, staged.data(), staged.size(), hipMemcpyHostToDevice,
+                               dev->stream));
+    HIP_TRY(st, hipStreamSynchronize(dev->stream));
+    reading.stream = nullptr;
+  }
   *out = p.release();
   return ORION_HIP_OK;
 }

@@ -1,6 +1,6 @@
-"""Fails each HIP call of a forward and of a sampler call in turn, on the fake
-runtime, and prints what was still queued when the call returned (the staging
-areas it reads are then overwritten or freed by the next call).
+"""Fails each HIP call of a forward, of a sampler call and of making a decode plan in
+turn, on the fake runtime, and prints what was still queued when the call returned
+(the staging areas it reads are then overwritten or freed).
 usage: errors_wait.py FAKE_HIP_LIBRARY"""
 import ctypes
 import os
@@ -55,10 +55,24 @@ def sample():
         be.close()
 
 
+def plan():
+    be = oh.HipBackend(0)
+    logits = be.alloc(1000 * 4)
+    try:
+        # (the sampler's pinned memory: from here on queued work is counted)
+        oh.sample(be, logits.ptr, 1, 1000, [oh.SamplingParams(temperature=1.0)],
+                  [np.array([], np.uint32)], np.full(1, 0.5, np.float32))
+        oh.DecodePlan(be, [299], np.zeros(1, np.int32), np.array([0, 19]), np.arange(19), 32, 4, 64,
+                      16).close()
+    finally:
+        results.append(fake.fake_hip_queued())
+        be.close()
+
+
 for name, run in [("decode 1 row", forward(decode(1, 40))),
                   ("decode 9 rows, then longer", forward(decode(9, 30), decode(40, 600))),
                   ("decode 96 rows", forward(decode(96, 100))),
-                  ("prompt", forward(prompt(300))), ("sample", sample)]:
+                  ("prompt", forward(prompt(300))), ("sample", sample), ("plan", plan)]:
     results = []
     fake.fake_hip_fail_at(0)
     run()

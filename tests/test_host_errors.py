@@ -20,14 +20,14 @@ def fake_hip(tmp_path_factory):
 
 
 def test_every_error_waits_for_the_staging_areas(fake_hip):
-    # each HIP call of a forward and a sampler call fails in turn: the call
-    # reports it, and no work that may read the pinned staging areas, which the
-    # next call writes, is still queued
+    # each HIP call of a forward, a sampler call and a plan's making fails in turn:
+    # the call reports it, and no work that may read the staging areas, which are
+    # then written or freed, is still queued
     p = subprocess.run([sys.executable, os.path.join(FAKE, "errors_wait.py"), fake_hip],
                        capture_output=True, text=True, timeout=300)
     assert p.returncode == 0, p.stderr
     lines = p.stdout.splitlines()
-    assert len(lines) == 5, p.stdout
+    assert len(lines) == 6, p.stdout
     for line in lines:
         calls, errors, left = [int(part.split()[0]) for part in line.split(": ")[1].split(", ")[:3]]
         assert calls == errors and left == 0, line
